@@ -211,8 +211,7 @@ int mugen_attn_gqa_decode_q4(const mugen_attn_gqa_decode_q4_args* args, void* wo
  *   causal = 0 lets every token see all kv_len keys.
  *
  * Supported: head_dim a multiple of 8 up to 256 (as gqa_decode; above 128
- * every query token attends in its own workgroup, the reference's per-token
- * CPU rule, and only kernel 0 is accepted);
+ * only kernel 0 is accepted);
  * n_heads / n_kv_heads in [1, 16] (more
  * than 8 runs on the warp-specialised kernel; forcing the per-block kernel
  * there is refused); dtype F16 or BF16 for q/k/v; out_dtype F16/BF16/F32.
@@ -269,8 +268,8 @@ int mugen_attn_gqa_prefill(const mugen_attn_gqa_prefill_args* args, void* stream
  * (kv_len * n_kv_heads * head_dim * 2 + 256 for BF16 prompts of at least
  * 1024 tokens and for some split calls, where the separate conversion pays
  * for its launch) plus the split partials (n_tokens * n_heads * splits *
- * (2 * head_dim + 8) + 512 when the key range is split), else 0 (also for
- * invalid args).  The size never falls as kv_len grows at a fixed n_tokens.
+ * (2 * head_dim + 8) + 512 when the key range is split, 4 * head_dim + 8
+ * above head_dim 128), else 0 (also for invalid args).  The size never falls as kv_len grows at a fixed n_tokens.
  * No counterpart in the reference (it runs each chunk on one pass over its
  * keys). */
 size_t mugen_attn_gqa_prefill_workspace_size(const mugen_attn_gqa_prefill_args* args);

@@ -18,7 +18,7 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 LIB_NAME = "libmugen_attn.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
-SOURCES = ["capi.hip", "engine.hip", "gqa_decode.hip", "gqa_prefill.hip", "kv_q4.hip", "mla_cache.hip",
+SOURCES = ["capi.hip", "engine.hip", "gqa_decode.hip", "gqa_prefill.hip", "gqa_prefill_rows.hip", "kv_q4.hip", "mla_cache.hip",
            "mla_decode.hip", "mla_proj.hip"]
 ARCH = "gfx950"
 

@@ -641,6 +641,13 @@ static bool gqa_prefill_v16_capable(const mugen_attn_gqa_prefill_args* a) {
     return a->head_dim <= 128 && a->dtype == DT_BF16;
 }
 
+// head_dim above 128, keys not split: up to this many (token, kv head) pairs
+// (one round of workgroups) run one to a workgroup, whose four waves share
+// the pair's keys; past it the flattened-row kernel.  16 / 8 heads, us,
+// per pair / flattened: N = 32 5.4 / 7.1, 64 9.9 / 8.5, 256 53 / 14.8; 16 / 4
+// heads at head_dim 192, N = 64 6.4 / 11.3, 512 86 / 26
+constexpr int kPrefillWideItems = 256;
+
 // The automatic choice of the short-prompt kernel: the whole kv range fits
 // on chip, from 384 visible keys on (below that the per-block kernel's
 // shorter load phase wins: Llama-3.2-1B N = 128 4.4 against 4.9 us; N = 256
@@ -662,17 +669,53 @@ static bool gqa_prefill_short_default(const mugen_attn_gqa_prefill_args* a) {
 // range: unsplit, workgroups for fewer than half the CUs walk the whole
 // range each.  Each block's keys are then split into ranges of whole steps
 // (at least kMinKeys, so that the partials' merge stays a small part of the
-// call) until the work list fills about one round; the partials (fp16
-// O / l, fp32 max and sum) go to the workspace after the fp16 V copy, and
+// call) until the work list fills about one round; the partials (O / l, fp16
+// up to head_dim 128 and fp32 above, fp32 max and sum) go to the workspace after the fp16 V copy, and
 // gqa_prefill_combine merges them.  The plan depends on the arguments only,
 // so the workspace size function and the call agree.
 struct PrefillSplit {
     int ksplit = 1, kchunk = 0;
     size_t bytes = 0;  // partial O and (max, sum) of every row and split
 };
+
+// The plan for `units` workgroups over steps of `step` keys: about `target`
+// workgroups, ranges of at least 256 keys; `part` bytes of partial per row
+static PrefillSplit prefill_split_plan(const mugen_attn_gqa_prefill_args* a, int64_t units, int64_t target, int step,
+                                       size_t part) {
+    PrefillSplit r;
+    const int kend = a->causal ? std::min(a->kv_len, a->start_pos + a->n_tokens) : a->kv_len;
+    const int steps = ceil_div(kend, step);
+    constexpr int kMinKeys = 256;
+    const int64_t want =
+        std::min<int64_t>({ceil_div(target, units), (int64_t)steps / (kMinKeys / step), (int64_t)kPrefillMaxSplits});
+    if (want < 2) return r;
+    const int kchunk = ceil_div(steps, (int)want) * step;
+    const int ks = ceil_div(kend, kchunk);
+    if (ks < 2) return r;
+    r.ksplit = ks;
+    r.kchunk = kchunk;
+    // sized for `want` ranges (ks <= want): want never falls as the key
+    // range grows, so the size at the longest range covers every shorter one
+    r.bytes = (size_t)a->n_tokens * a->n_heads * want * (part + 2 * sizeof(float)) + 512;
+    return r;
+}
+
 static PrefillSplit gqa_prefill_split(const mugen_attn_gqa_prefill_args* a) {
     PrefillSplit r;
-    if (a->head_dim > 128 || a->n_tokens <= 0 || a->kv_len <= 0) return r;
+    if (a->n_tokens <= 0 || a->kv_len <= 0) return r;
+    if (a->head_dim > 128) {
+        // the flattened-row kernel, one workgroup per CU, fp32 partials: chunks
+        // that follow a context (16 / 8 heads: 5 / 100 / 300 tokens after 1500
+        // 43 / 55 / 62 us unsplit, 17 / 26 / 32 split).  A prompt from
+        // position 0 has long ranges in few of its rows, and every row's
+        // partials to store and merge: 512 tokens 22.6 us unsplit, 28.7 split,
+        // 1021 tokens 38.4 and 37.8
+        const int64_t blocks = ((int64_t)a->n_tokens * (a->n_heads / a->n_kv_heads) + 127) / 128;
+        const int64_t units = blocks * a->n_kv_heads;
+        const int keys = a->causal ? std::min(a->kv_len, a->start_pos + a->n_tokens) : a->kv_len;
+        if (units * 2 > 256 || keys < (int64_t)a->n_tokens + 640) return r;
+        return prefill_split_plan(a, units, 256, 32, (size_t)a->head_dim * 4);
+    }
     if (a->kernel && a->kernel != MUGEN_ATTN_PREFILL_KERNEL_WS) return r;
     if (!a->kernel && gqa_prefill_short_default(a)) return r;  // every key on chip already
     const int G = a->n_heads / a->n_kv_heads;
@@ -692,23 +735,10 @@ static PrefillSplit gqa_prefill_split(const mugen_attn_gqa_prefill_args* a) {
     // over long ranges: H32 Hk8 d64, 256 tokens after 1024 measured 15.0
     // split against 13.9 us, after 2048 19.3 against 23.4
     if (G <= 4 && units * 4 > 256 && kend < 2048) return r;
-    const int steps = ceil_div(kend, step);
     // ranges of at least 256 keys (4 steps of 64, 8 of 32): verify-sized
     // chunks (5 tokens after 4000, 7B shape) 18.1 -> 13.8 us against 512
     // keys; 4-head blocks at 128 keys measured slower (9.2 -> 10.3 us)
-    constexpr int kMinKeys = 256;
-    const int64_t want =
-        std::min<int64_t>({ceil_div(target, units), (int64_t)steps / (kMinKeys / step), (int64_t)kPrefillMaxSplits});
-    if (want < 2) return r;
-    const int kchunk = ceil_div(steps, (int)want) * step;
-    const int ks = ceil_div(kend, kchunk);
-    if (ks < 2) return r;
-    r.ksplit = ks;
-    r.kchunk = kchunk;
-    // sized for `want` ranges (ks <= want): want never falls as the key
-    // range grows, so the size at the longest range covers every shorter one
-    r.bytes = (size_t)a->n_tokens * a->n_heads * want * (a->head_dim * 2 + 2 * sizeof(float)) + 512;
-    return r;
+    return prefill_split_plan(a, units, target, step, (size_t)a->head_dim * 2);
 }
 
 // The fp16 copy of V (one extra launch over kv_len rows): for long BF16
@@ -734,12 +764,41 @@ size_t mugen_attn_gqa_prefill_workspace_size(const mugen_attn_gqa_prefill_args* 
 int mugen_attn_gqa_prefill(const mugen_attn_gqa_prefill_args* a, void* stream) {
     if (int rc = gqa_prefill_validate(a)) return rc;
     if (a->n_tokens == 0) return MUGEN_ATTN_OK;
+    GqaPrefillParams p{};
+    p.q = static_cast<const uint16_t*>(a->q);
+    p.k = static_cast<const uint16_t*>(a->k);
+    p.v = static_cast<const uint16_t*>(a->v);
+    p.out = a->out;
+    p.N = a->n_tokens;
+    p.H = a->n_heads;
+    p.G = a->n_heads / a->n_kv_heads;
+    p.hd = a->head_dim;
+    p.row_stride = a->n_kv_heads * a->head_dim;
+    p.kv_len = a->kv_len;
+    p.start_pos = a->start_pos;
+    p.causal = a->causal ? 1 : 0;
+    const float scale = a->scale > 0.f ? a->scale : 1.f / sqrtf((float)a->head_dim);
+    p.scale_log2 = scale * kLog2e;
     if (a->head_dim > 128) {
-        // head_dim 129..256: the per-token rule of the reference's CPU path
+        if (a->kernel) return fail(MUGEN_ATTN_E_UNSUPPORTED, "gqa_prefill: head_dim > 128 has one kernel (kernel 0)");
+        hipStream_t st = static_cast<hipStream_t>(stream);
+        const PrefillSplit split = gqa_prefill_split(a);
+        p.ksplit = 1;
+        if (split.ksplit > 1 && a->workspace && a->workspace_bytes >= split.bytes) {
+            p.ksplit = split.ksplit;
+            p.kchunk = split.kchunk;
+            p.ws_ml = align256(a->workspace);
+            p.ws_o = reinterpret_cast<uint16_t*>(p.ws_ml + (size_t)a->n_tokens * a->n_heads * split.ksplit * 2);
+        }
+        if (p.ksplit > 1 || (int64_t)a->n_tokens * a->n_kv_heads > kPrefillWideItems) {
+            hipError_t e = launch_gqa_prefill_rows(p, a->n_kv_heads, a->dtype, a->out_dtype, st, active_timer());
+            if (e == hipSuccess && p.ksplit > 1) e = launch_gqa_prefill_combine(p, a->out_dtype, st, active_timer());
+            return hip_status(e, "gqa_prefill launch");
+        }
+        // a few tokens, unsplit: the per-token rule of the reference's CPU path
         // (query i of the prompt attends over start_pos + i + 1 keys,
         // transformer.cpp:1334-1335) on the decode kernel's prompt mode, one
         // (token, kv head) per workgroup over the shared cache
-        if (a->kernel) return fail(MUGEN_ATTN_E_UNSUPPORTED, "gqa_prefill: head_dim > 128 has one kernel (kernel 0)");
         GqaDecodeParams d{};
         d.B = a->n_tokens;
         d.Hk = a->n_kv_heads;
@@ -760,25 +819,9 @@ int mugen_attn_gqa_prefill(const mugen_attn_gqa_prefill_args* a, void* stream) {
         d.pf_causal = a->causal ? 1 : 0;
         if ((int64_t)a->n_tokens * a->n_kv_heads > INT32_MAX)
             return fail(MUGEN_ATTN_E_UNSUPPORTED, "gqa_prefill: n_tokens * n_kv_heads too large");
-        return hip_status(launch_gqa_prefill_wide(d, a->dtype, a->out_dtype, static_cast<hipStream_t>(stream),
-                                                  active_timer()),
+        return hip_status(launch_gqa_prefill_wide(d, a->dtype, a->out_dtype, st, active_timer()),
                           "gqa_prefill launch");
     }
-    GqaPrefillParams p{};
-    p.q = static_cast<const uint16_t*>(a->q);
-    p.k = static_cast<const uint16_t*>(a->k);
-    p.v = static_cast<const uint16_t*>(a->v);
-    p.out = a->out;
-    p.N = a->n_tokens;
-    p.H = a->n_heads;
-    p.G = a->n_heads / a->n_kv_heads;
-    p.hd = a->head_dim;
-    p.row_stride = a->n_kv_heads * a->head_dim;
-    p.kv_len = a->kv_len;
-    p.start_pos = a->start_pos;
-    p.causal = a->causal ? 1 : 0;
-    const float scale = a->scale > 0.f ? a->scale : 1.f / sqrtf((float)a->head_dim);
-    p.scale_log2 = scale * kLog2e;
     // the warp-specialised kernel where it measured faster: every prompt
     // above head_dim 64 (graph replays: Qwen2.5-7B shape N = 16 / 256 / 768
     // 5.9 / 10.7 / 21.6 against 7.5 / 11.9 / 22.4 us, H32 Hk8 d128 N = 768

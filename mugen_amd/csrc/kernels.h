@@ -114,7 +114,8 @@ struct GqaPrefillParams {
     int hd;          // head_dim of q, the caches and out (<= D, a multiple of 8)
     // key splits (warp-specialised kernel; 1 = none): workgroup split s takes
     // keys [s kchunk, (s+1) kchunk) of its query block and writes the rows'
-    // normalised partial O (O_s / l_s, fp16) to ws_o [N][H][ksplit][hd] and
+    // normalised partial O (O_s / l_s, fp16; fp32 above head_dim 128, where
+    // ws_o points to floats) to ws_o [N][H][ksplit][hd] and
     // (reference max in log2 units, weight sum l_s) to ws_ml
     // [N][H][ksplit][2]; the gqa_prefill_combine kernel then merges them
     // into out
@@ -129,6 +130,13 @@ struct GqaPrefillParams {
 // S / PV waves
 hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int Hk, int D, int dt, int out_dt, int kernel,
                               hipStream_t st, KernelTimer* t);
+// 128-row blocks of flattened (token, head) rows (gqa_prefill_rows.hip),
+// head_dim above 128; with p.ksplit > 1 the partials only (the caller merges
+// them)
+hipError_t launch_gqa_prefill_rows(const GqaPrefillParams& p, int Hk, int dt, int out_dt, hipStream_t st,
+                                   KernelTimer* t);
+// merge of the key splits' partials (fp16 up to head_dim 128, fp32 above)
+hipError_t launch_gqa_prefill_combine(const GqaPrefillParams& p, int out_dt, hipStream_t st, KernelTimer* t);
 // kernel 3 (MUGEN_ATTN_PREFILL_KERNEL_SHORT): every key a query block sees
 // held in LDS; serves head_dim 64 (unpadded), at most 4 heads per kv head
 // and a kv range (start_pos + N causal, kv_len otherwise) of at most 512
