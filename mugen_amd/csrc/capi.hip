@@ -641,6 +641,20 @@ static bool gqa_prefill_v16_capable(const mugen_attn_gqa_prefill_args* a) {
     return a->head_dim <= 128 && a->dtype == DT_BF16;
 }
 
+// head_dim up to 128: the flattened-row kernel where its 128-row blocks make
+// enough workgroups (two share a CU, three at head_dim 64) that the longest
+// causal rows' chain does not set the time.  us, before (warp-specialised or
+// per-block) / flattened: 28 / 4 heads d128 448 workgroups (N = 2048) 42.3 / 47.9,
+// 672 90 / 82; 16 / 2 d128 512 77 / 94; 32 / 8 d128 512 52.5 / 50.7; d64 512 34.0 /
+// 37.0, 768 66 / 58; 14 / 2 d64 448 49 / 63, 656 105 / 98.  At 1 or 2 heads per kv head the 4-head blocks
+// of the warp-specialised kernel are at most half full: from 256 workgroups
+// (8 / 8 d128 129 / 83, 128 workgroups 40 / 44; 16 / 16 d64 256 43 / 34)
+static bool gqa_prefill_rows_default(const mugen_attn_gqa_prefill_args* a) {
+    const int G = a->n_heads / a->n_kv_heads;
+    const int64_t wgs = ((int64_t)a->n_tokens * G + 127) / 128 * a->n_kv_heads;
+    return wgs >= (G <= 2 ? 256 : G <= 4 && a->head_dim > 64 ? 512 : 640);
+}
+
 // head_dim above 128, keys not split: up to this many (token, kv head) pairs
 // (one round of workgroups) run one to a workgroup, whose four waves share
 // the pair's keys; past it the flattened-row kernel.  16 / 8 heads, us,
@@ -822,23 +836,20 @@ int mugen_attn_gqa_prefill(const mugen_attn_gqa_prefill_args* a, void* stream) {
         return hip_status(launch_gqa_prefill_wide(d, a->dtype, a->out_dtype, st, active_timer()),
                           "gqa_prefill launch");
     }
-    // the warp-specialised kernel where it measured faster: every prompt
-    // above head_dim 64 (graph replays: Qwen2.5-7B shape N = 16 / 256 / 768
-    // 5.9 / 10.7 / 21.6 against 7.5 / 11.9 / 22.4 us, H32 Hk8 d128 N = 768
-    // 18.0 against 26.5; eager: N = 8192 603 against 690 us, 32768 8.76
-    // against 8.86 ms), at head_dim 64 from 1024 to 4096 tokens (Llama-3.2-1B
-    // shape N = 4096 114 against 116 us, N = 8192 423 against 381; below 1024
-    // the per-block and short-prompt kernels lead: N = 512 7.7 against 9.2);
-    // args->kernel forces one.  At head_dim 64 the limits above are the
-    // 4-head blocks' (G <= 4); its 8-head blocks (G > 4) lead at every length
-    // (H28 Hk4 d64 N = 6144 203 against 245 us, H16 Hk2 N = 256 7.4 against
-    // 8.0; within 1 us either way at N = 512)
+    // below the flattened-row kernel's sizes: the warp-specialised kernel above
+    // head_dim 64 and for more than 4 heads per kv head (graph replays, us:
+    // Qwen2.5-7B shape N = 16 / 256 / 768 5.9 / 10.7 / 21.6 against 7.5 / 11.9 /
+    // 22.4 per-block, H32 Hk8 d128 N = 768 18.0 against 26.5; H16 Hk2 d64 N = 256
+    // 7.4 against 8.0); 4-head blocks at head_dim 64 from 1024 tokens (below, the
+    // per-block and short-prompt kernels lead: N = 512 7.7 against 9.2).
+    // args->kernel forces one
     const bool ws_default =
-        a->head_dim > 64 || p.G > 4 || (a->n_tokens >= 1024 && a->n_tokens <= 4096);
+        a->head_dim > 64 || p.G > 4 || a->n_tokens >= 1024;
     int kernel = ws_default ? MUGEN_ATTN_PREFILL_KERNEL_WS : MUGEN_ATTN_PREFILL_KERNEL_BLOCK;
     // prompts whose whole kv range fits on chip: the short-prompt kernel
     const bool short_fits = gqa_prefill_short_fits(p, padded_head_dim(a->head_dim));
     if (gqa_prefill_short_default(a)) kernel = MUGEN_ATTN_PREFILL_KERNEL_SHORT;
+    const bool rows = !a->kernel && kernel != MUGEN_ATTN_PREFILL_KERNEL_SHORT && gqa_prefill_rows_default(a);
     if (a->kernel == MUGEN_ATTN_PREFILL_KERNEL_SHORT && !short_fits)
         return fail(MUGEN_ATTN_E_UNSUPPORTED,
                     "gqa_prefill: the short kernel serves head_dim 64, n_heads/n_kv_heads <= 4 and <= 512 keys");
@@ -865,8 +876,11 @@ int mugen_attn_gqa_prefill(const mugen_attn_gqa_prefill_args* a, void* stream) {
         p.v = v16;
         dt = kDtBf16V16;
     }
-    hipError_t e = launch_gqa_prefill(p, a->n_kv_heads, padded_head_dim(a->head_dim), dt, a->out_dtype, kernel,
-                                      static_cast<hipStream_t>(stream), active_timer());
+    hipError_t e = rows && p.ksplit == 1
+                       ? launch_gqa_prefill_rows(p, a->n_kv_heads, dt, a->out_dtype, static_cast<hipStream_t>(stream),
+                                                 active_timer())
+                       : launch_gqa_prefill(p, a->n_kv_heads, padded_head_dim(a->head_dim), dt, a->out_dtype, kernel,
+                                            static_cast<hipStream_t>(stream), active_timer());
     return hip_status(e, "gqa_prefill launch");
 }
 

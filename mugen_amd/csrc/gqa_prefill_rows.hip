@@ -30,7 +30,19 @@
 //    of tile j - 1 and computes S(j + 1) beside the softmax of tile j, so a
 //    wave's MFMAs, LDS reads and VALU work overlap inside the wave.
 //
-// Bound: MFMA issue of one wave per SIMD at head_dim 256 (64 MFMAs of 32
+// Bound up to head_dim 128 (two waves per SIMD): the SIMDs' issue slots -- per
+// 32-key tile and 32 rows 16 MFMAs of 32 cycles and ~80 VALU instructions at
+// head_dim 128, ~0.51 us per tile and wave against 0.26 of MFMAs; leaving out
+// the DMA, the LDS reads or the softmax takes 14 / 10 / 9% off (timing builds).
+// Against the warp-specialised kernel (gqa_prefill.hip), f16, us: 28 / 4 heads
+// at head_dim 128 N = 3072 / 4096 / 8192 90 / 148 / 557 -> 82 / 132 / 490, 8 / 8
+// heads N = 4096 129 -> 83, 32 / 8 heads at head_dim 64 (bf16) N = 4096 / 8192
+// 107 / 391 -> 84 / 300.
+// Blocks of 256 rows (8 waves, a 10-slot ring) measured the same, and constant
+// ring slots (the loop unrolled over the ring) 1% faster at N = 8192 for four
+// times the code.
+//
+// Bound at head_dim 256: MFMA issue of one wave per SIMD (64 MFMAs of 32
 // cycles per 64 keys and 32 rows), ~1.3 us per pair of tiles measured against
 // 0.9 of MFMAs.  16 / 8 heads, f16, one prompt: N = 1021 523 -> 38 us (16 ->
 // 226 TFLOP/s), N = 2048 1890 -> 70 us, 100 tokens after 1500 172 -> 26 us;
@@ -507,9 +519,10 @@ static hipError_t launch_rows_t(const GqaPrefillParams& p, int Hk, hipStream_t s
     const int groups = Hk * (p.ksplit > 1 ? p.ksplit : 1);
     // (the kernel's deal of blocks to XCDs)
     const int grid = groups < 8 && 8 % groups == 0 ? 8 * ((nblk * groups + 7) / 8) : nblk * groups;
-    if (p.ksplit > 1)
-        return launch_k(t, "gqa_prefill", gqa_prefill_rows_kernel<D, DT, DT_F32, PAD, true>, dim3(grid), dim3(256), st,
-                        p, nblk, Hk);
+    if constexpr (D > 128)
+        if (p.ksplit > 1)
+            return launch_k(t, "gqa_prefill", gqa_prefill_rows_kernel<D, DT, DT_F32, PAD, true>, dim3(grid), dim3(256),
+                            st, p, nblk, Hk);
     return launch_k(t, "gqa_prefill", gqa_prefill_rows_kernel<D, DT, OUT_DT, PAD, false>, dim3(grid), dim3(256), st, p,
                     nblk, Hk);
 }
@@ -531,9 +544,15 @@ static hipError_t launch_rows_d(const GqaPrefillParams& p, int Hk, int dt, int o
 
 hipError_t launch_gqa_prefill_rows(const GqaPrefillParams& p, int Hk, int dt, int out_dt, hipStream_t st,
                                    KernelTimer* t) {
-    if (p.hd <= 128) return hipErrorInvalidValue;  // served by gqa_prefill.hip
-    return p.hd != 256 ? launch_rows_d<256, true>(p, Hk, dt, out_dt, st, t)
-                       : launch_rows_d<256, false>(p, Hk, dt, out_dt, st, t);
+    if (p.hd > 128)
+        return p.hd != 256 ? launch_rows_d<256, true>(p, Hk, dt, out_dt, st, t)
+                           : launch_rows_d<256, false>(p, Hk, dt, out_dt, st, t);
+    if (p.ksplit > 1) return hipErrorInvalidValue;  // split ranges: the warp-specialised kernel
+    if (p.hd > 64)
+        return p.hd != 128 ? launch_rows_d<128, true>(p, Hk, dt, out_dt, st, t)
+                           : launch_rows_d<128, false>(p, Hk, dt, out_dt, st, t);
+    return p.hd != 64 ? launch_rows_d<64, true>(p, Hk, dt, out_dt, st, t)
+                      : launch_rows_d<64, false>(p, Hk, dt, out_dt, st, t);
 }
 
 }  // namespace mugen_attn

@@ -130,8 +130,8 @@ struct GqaPrefillParams {
 // S / PV waves
 hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int Hk, int D, int dt, int out_dt, int kernel,
                               hipStream_t st, KernelTimer* t);
-// 128-row blocks of flattened (token, head) rows (gqa_prefill_rows.hip),
-// head_dim above 128; with p.ksplit > 1 the partials only (the caller merges
+// 128-row blocks of flattened (token, head) rows (gqa_prefill_rows.hip); with
+// p.ksplit > 1 (head_dim above 128 only) the partials only (the caller merges
 // them)
 hipError_t launch_gqa_prefill_rows(const GqaPrefillParams& p, int Hk, int dt, int out_dt, hipStream_t st,
                                    KernelTimer* t);

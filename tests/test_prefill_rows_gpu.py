@@ -62,6 +62,32 @@ def test_wide_rows_split(device, N, H, Hk, D, start, dtype):
     check(c, device, f"split rows N={N} D={D} start={start}, 16-bit output", dtype)
 
 
+# head_dim up to 128: just past the workgroup counts where this kernel takes
+# over (256 at 1 or 2 heads per kv head, 512 up to 4 above head_dim 64, else 640),
+# with and without the fp16 copy of V.  The first rows, a stretch in the middle
+# and the last rows, through the oracle's start-offset form
+NARROW = [(2926, 28, 4, 128, 0), (1640, 40, 10, 96, 0), (1030, 32, 32, 128, 0), (1900, 33, 11, 64, 5),
+          (3300, 16, 8, 64, 0), (860, 96, 16, 48, 3)]
+
+
+@pytest.mark.parametrize("N,H,Hk,D,start", NARROW)
+@pytest.mark.parametrize("dtype", [C.F16, C.BF16])
+def test_narrow_rows(device, N, H, Hk, D, start, dtype):
+    c = C.prefill_case(1600 + N + D, N, H, Hk, D, start, dtype)
+    for passes in (0, 1) if dtype == C.BF16 else (0,):
+        if passes == 0:
+            got, _ = run(c, device)
+        else:  # no workspace: V converted on chip
+            q, k, v = (C.to_dev(c[x], dtype, device) for x in ("qb", "kb", "vb"))
+            got = mugen_amd.flash_prefill_attention(q, k, v, start, out_dtype=torch.float32,
+                                                    workspace=torch.empty(0, dtype=torch.uint8, device=device))
+            got = got.cpu().numpy()
+        for lo, n in ((0, 40), (N // 2 - 20, 40), (N - 40, 40)):
+            kv = start + lo + n
+            ref = C.O.gqa_prefill(c["q"][lo:lo + n], c["k"][:kv], c["v"][:kv], n, H, Hk, D, kv, start + lo, nthreads=16)
+            C.assert_close(got[lo:lo + n], ref, f"rows N={N} D={D} rows {lo}..{lo + n}")
+
+
 def test_wide_rows_not_causal(device):
     c = C.prefill_case(1400, 140, 8, 4, 256, 53, C.F16)
     got, _ = run(c, device, causal=False)
@@ -71,14 +97,15 @@ def test_wide_rows_not_causal(device):
     C.assert_close(got, ref, "rows, not causal")
 
 
+@pytest.mark.parametrize("N,H,Hk,D", [(200, 8, 2, 256), (300, 96, 96, 128), (300, 96, 96, 64)])
 @pytest.mark.parametrize("dtype", [C.F16, C.BF16])
-def test_wide_rows_climbing_scores(device, dtype):
-    # scores that climb by > 15 log2 units per tile: the re-base runs on every
-    # tile.  The same inputs as the other kernels' test, scaled for head_dim 256
-    c = C.prefill_case(1500, 200, 8, 2, 256, 20, dtype)
+def test_rows_climbing_scores(device, N, H, Hk, D, dtype):
+    # scores that climb by > 11 log2 units per tile: rows re-base again and
+    # again.  The other kernels' inputs, q scaled with sqrt(head_dim)
+    c = C.prefill_case(1500 + D, N, H, Hk, D, 20, dtype)
     q, k = c["q"].copy(), c["k"].copy()
-    q[:, :, 0] = 16.0
+    q[:, :, 0] = 16.0 if D == 256 else 8.0
     k[:, :, 0] = 0.5 * np.arange(c["kv_len"], dtype=np.float32)[:, None]
     c["q"], c["qb"] = C.O.round_to(q, dtype)
     c["k"], c["kb"] = C.O.round_to(k, dtype)
-    check(c, device, "climbing scores, head_dim 256")
+    check(c, device, f"climbing scores, head_dim {D}")
