@@ -183,6 +183,8 @@ constexpr int kPlanSplitCap = 32, kGqaChunkMin = 64;
 // -> 18.2 us.  The 32-way cap (with the floor lowered from 128 to 64
 // tokens): B1 T2048 7.38 -> 6.87 us, T8192 10.83 -> 9.17, B2 T8192 12.98
 // -> 10.0; B16 and B1 T4096 unchanged (their plans were ~32 splits).
+static int gqa_budget(const mugen_attn_gqa_decode_args* a) { return a->head_dim > 128 ? 256 : 512; }
+
 static int gqa_chunk(const mugen_attn_gqa_decode_args* a, int extra = 0) {
     constexpr int q = 32, qmin = kGqaChunkMin, kSplitCap = kPlanSplitCap;
     const int maxT = a->max_seq_len > 0 ? a->max_seq_len : 1;
@@ -199,7 +201,7 @@ static int gqa_chunk(const mugen_attn_gqa_decode_args* a, int extra = 0) {
     const int cmin = std::max(ceil_div(ceil_div(maxT, kMaxSplits - 1), q), ceil_div(ceil_div(tlong, kSplitCap), q)) * q;
     // one dispatch round: two workgroups per CU, one at head_dim 256 (one
     // wave per SIMD)
-    const int64_t budget = a->head_dim > 128 ? 256 : 512;
+    const int64_t budget = gqa_budget(a);
     if (gqa_items(a, cmax, extra) > budget) return cmax;  // one split per sequence already fills a round
     int lo = cmin < qmin ? qmin : cmin, hi = cmax;        // items(c) is non-increasing in c
     while (lo < hi) {
@@ -274,6 +276,31 @@ static int stride_bound(int max_seq_len, int qmin, int extra) {
     return std::min(kPlanSplitCap, ceil_div(maxT, qmin)) + extra;
 }
 
+// Without host lengths (a captured step, replayed as its sequences grow) the
+// kernels plan the chunk from the device lengths: a plan made for max_seq_len
+// cuts a cache that is not full into too few splits (16 ragged sequences of up
+// to 4096 tokens in 8192-token caches, 28 / 4 heads: 273 of 512 workgroups had
+// work).  The longest sequence gets as many splits as the workspace has room
+// for, up to stride_bound, which the workspace sizes cover; below the static
+// plan's own count, and in large batches, whose sequences fill half a round
+// unsplit, the static plan stays; also where its chunk is 128 tokens or less
+// (one sequence of 700 tokens in a 4096-token cache: 6.0 us static, 6.2 planned,
+// of 3000 in 8192, chunk 256: 8.9 and 7.5).
+static bool gqa_device_plan(const mugen_attn_gqa_decode_args* a, int extra) {
+    return !a->seq_lens_host && a->num_splits <= 0 && (int64_t)a->batch * a->n_kv_heads * 2 <= gqa_budget(a) &&
+           stride_bound(a->max_seq_len, kGqaChunkMin, extra) > 1;
+}
+constexpr int kPlanStaticChunk = 128;
+constexpr size_t kPlanBytes = 256;  // the planned chunk, after the partials
+// most splits per sequence whose partials (one split's: `per` bytes) fit a
+// workspace beside the alignment and the plan
+static int plan_fit(size_t ws_bytes, size_t per, int bound) {
+    return ws_bytes < 256 + kPlanBytes ? 0 : (int)std::min<size_t>((ws_bytes - 256 - kPlanBytes) / per, bound);
+}
+static size_t gqa_split_bytes(const mugen_attn_gqa_decode_args* a) {
+    return (size_t)a->batch * a->n_heads * ((size_t)padded_head_dim(a->head_dim) * 4 + 8);
+}
+
 static size_t gqa_ws(const mugen_attn_gqa_decode_args* a, int chunk, int* splits_out, int min_splits = 0) {
     const int splits = std::max(plan_stride(a->max_seq_len, chunk, a->seq_lens_host, a->batch, 0), min_splits);
     if (splits_out) *splits_out = splits;
@@ -323,6 +350,7 @@ static int64_t mla_units(const mugen_attn_mla_decode_args* a, int chunk, int64_t
 // the smallest chunk (multiple of 32) whose nrb * active groups fit ONE
 // dispatch round of 256 CUs -- maximum parallelism, no second round -- with
 // the longest sequence split at most 32 ways.
+constexpr int kMlaBudget = 256;
 static int mla_chunk(const mugen_attn_mla_decode_args* a, int kernel) {
     const int q = mla_tile_tokens(kernel);  // chunks are whole tiles
     if (a->num_splits > 0) return explicit_chunk(a->max_seq_len, a->num_splits, q, kMaxMlaSplits);
@@ -342,7 +370,7 @@ static int mla_chunk(const mugen_attn_mla_decode_args* a, int kernel) {
         for (int b = 0; b < a->batch; b++) tlong = std::max(tlong, std::min(a->seq_lens_host[b], maxT));
     }
     const int cmin = std::max(ceil_div(ceil_div(maxT, kMaxMlaSplits), q), ceil_div(ceil_div(tlong, kSplitCap), q)) * q;
-    const int64_t wg_budget = 256;
+    const int64_t wg_budget = kMlaBudget;
     if (mla_units(a, cmax, nrb) > wg_budget) return cmax;  // one split per sequence already fills a round
     int lo = cmin < q ? q : cmin, hi = cmax;               // units(c) is non-increasing in c
     while (lo < hi) {
@@ -391,6 +419,18 @@ static size_t mla_ws(const mugen_attn_mla_decode_args* a, int chunk, int* splits
     const size_t rows16 = (R + 15) / 16 * 16;  // O partials are stored per 16-row block
     const size_t sb = (size_t)a->batch * splits;
     return sb * rows16 * 512 * 2 + sb * R * 2 * 4 + 256;
+}
+
+// As gqa_device_plan, for decode and verify steps (a prompt's plan counts the
+// causal units and stays on the host); a workspace without room for every
+// plan's partials keeps the plan for max_seq_len
+static bool mla_device_plan(const mugen_attn_mla_decode_args* a, int kernel) {
+    const int nrb = ceil_div((int64_t)a->q_len * a->n_heads, mla_rows_per_block(kernel));
+    return !a->seq_lens_host && a->num_splits <= 0 && a->q_len <= 16 && (int64_t)a->batch * nrb * 2 <= kMlaBudget;
+}
+static size_t mla_split_bytes(const mugen_attn_mla_decode_args* a) {
+    const size_t R = (size_t)a->q_len * a->n_heads;
+    return (size_t)a->batch * ((R + 15) / 16 * 16 * 512 * 2 + R * 8);
 }
 
 static float* align256(void* p) {
@@ -505,7 +545,7 @@ size_t mugen_attn_gqa_decode_q4_workspace_size(const mugen_attn_gqa_decode_q4_ar
     if (gqa_q4_validate(a) != MUGEN_ATTN_OK) return 0;
     const mugen_attn_gqa_decode_args g = q4_as_gqa(a);
     const int bound = (!a->seq_lens_host && a->num_splits <= 0) ? stride_bound(a->max_seq_len, kGqaChunkMin, 1) : 0;
-    return gqa_q4_ws(a, gqa_chunk(&g, 1), nullptr, bound);
+    return gqa_q4_ws(a, gqa_chunk(&g, 1), nullptr, bound) + (gqa_device_plan(&g, 1) ? kPlanBytes : 0);
 }
 
 int mugen_attn_gqa_decode_q4(const mugen_attn_gqa_decode_q4_args* a, void* ws, size_t ws_bytes, void* stream) {
@@ -513,7 +553,10 @@ int mugen_attn_gqa_decode_q4(const mugen_attn_gqa_decode_q4_args* a, void* ws, s
     const mugen_attn_gqa_decode_args g = q4_as_gqa(a);
     const int chunk = gqa_chunk(&g, 1);
     int splits = 2;
-    const size_t need = gqa_q4_ws(a, chunk, &splits);
+    size_t need = gqa_q4_ws(a, chunk, &splits);
+    const int fit = ws ? plan_fit(ws_bytes, gqa_split_bytes(&g), stride_bound(a->max_seq_len, kGqaChunkMin, 1)) : 0;
+    const bool dev = gqa_device_plan(&g, 1) && chunk > kPlanStaticChunk && fit >= splits;
+    if (dev) need = gqa_q4_ws(a, chunk, &splits, fit);
     if (!ws || ws_bytes < need)
         return fail(MUGEN_ATTN_E_WORKSPACE, "gqa_decode_q4: workspace of %zu bytes required, %zu given", need,
                     ws_bytes);
@@ -546,8 +589,14 @@ int mugen_attn_gqa_decode_q4(const mugen_attn_gqa_decode_q4_args* a, void* ws, s
         const size_t slots = (size_t)a->batch * a->n_heads * splits;
         p.ws_o = base;
         p.ws_ml = base + slots * padded_head_dim(a->head_dim);
+        p.plan = reinterpret_cast<int*>(p.ws_ml + slots * 2);
     }
-    const int64_t nwg = gqa_items(&g, chunk, 1);  // + the ring splits
+    int64_t nwg = gqa_items(&g, chunk, 1);  // + the ring splits
+    if (dev) {
+        p.chunk = 0;
+        p.budget = gqa_budget(&g);
+        nwg = std::min<int64_t>(p.budget, (int64_t)a->batch * a->n_kv_heads * splits);
+    }
     if (nwg > INT32_MAX / 2) return fail(MUGEN_ATTN_E_UNSUPPORTED, "gqa_decode_q4: too many work items");
     p.per_xcd = (int)ceil_div(nwg, (int64_t)8);
     return hip_status(launch_gqa_decode_q4(p, (int)nwg, a->head_dim, a->out_dtype, static_cast<hipStream_t>(stream),
@@ -558,7 +607,7 @@ int mugen_attn_gqa_decode_q4(const mugen_attn_gqa_decode_q4_args* a, void* ws, s
 size_t mugen_attn_gqa_decode_workspace_size(const mugen_attn_gqa_decode_args* a) {
     if (gqa_validate(a) != MUGEN_ATTN_OK) return 0;
     const int bound = (!a->seq_lens_host && a->num_splits <= 0) ? stride_bound(a->max_seq_len, kGqaChunkMin, 0) : 0;
-    return gqa_ws(a, gqa_chunk(a), nullptr, bound);
+    return gqa_ws(a, gqa_chunk(a), nullptr, bound) + (gqa_device_plan(a, 0) ? kPlanBytes : 0);
 }
 
 int mugen_attn_gqa_decode(const mugen_attn_gqa_decode_args* a, void* ws, size_t ws_bytes, void* stream) {
@@ -566,7 +615,10 @@ int mugen_attn_gqa_decode(const mugen_attn_gqa_decode_args* a, void* ws, size_t 
     if (rc) return rc;
     const int chunk = gqa_chunk(a);
     int splits = 1;
-    const size_t need = gqa_ws(a, chunk, &splits);
+    size_t need = gqa_ws(a, chunk, &splits);
+    const int fit = ws ? plan_fit(ws_bytes, gqa_split_bytes(a), stride_bound(a->max_seq_len, kGqaChunkMin, 0)) : 0;
+    const bool dev = gqa_device_plan(a, 0) && chunk > kPlanStaticChunk && fit > 1 && fit >= splits;
+    if (dev) need = gqa_ws(a, chunk, &splits, fit);
     if (need > 0 && (!ws || ws_bytes < need))
         return fail(MUGEN_ATTN_E_WORKSPACE, "gqa_decode: workspace of %zu bytes required, %zu given", need,
                     ws_bytes);
@@ -593,8 +645,14 @@ int mugen_attn_gqa_decode(const mugen_attn_gqa_decode_args* a, void* ws, size_t 
         const size_t slots = (size_t)a->batch * a->n_heads * splits;
         p.ws_o = base;
         p.ws_ml = base + slots * padded_head_dim(a->head_dim);
+        p.plan = reinterpret_cast<int*>(p.ws_ml + slots * 2);
     }
-    const int64_t nwg = gqa_items(a, chunk);
+    int64_t nwg = gqa_items(a, chunk);
+    if (dev) {
+        p.chunk = 0;
+        p.budget = gqa_budget(a);
+        nwg = std::min<int64_t>(p.budget, (int64_t)a->batch * a->n_kv_heads * splits);
+    }
     if (nwg > INT32_MAX) return fail(MUGEN_ATTN_E_UNSUPPORTED, "gqa_decode: too many work items");
     hipError_t e = launch_gqa_decode(p, (int)nwg, padded_head_dim(a->head_dim), a->kv_dtype, a->out_dtype,
                                      static_cast<hipStream_t>(stream), active_timer());
@@ -889,7 +947,7 @@ size_t mugen_attn_mla_decode_workspace_size(const mugen_attn_mla_decode_args* a)
     const int bound = (!a->seq_lens_host && a->num_splits <= 0)
                           ? stride_bound(a->max_seq_len, mla_tile_tokens(mla_kernel(a)), 0)
                           : 0;
-    return mla_ws(a, mla_chunk(a, mla_kernel(a)), nullptr, bound);
+    return mla_ws(a, mla_chunk(a, mla_kernel(a)), nullptr, bound) + (mla_device_plan(a, mla_kernel(a)) ? kPlanBytes : 0);
 }
 
 }  // extern "C"
@@ -901,7 +959,10 @@ static int mla_decode_impl(const mugen_attn_mla_decode_args* a, void* ws, size_t
     const int kernel = mla_kernel(a);
     const int chunk = mla_chunk(a, kernel);
     int splits = 1;
-    const size_t need = mla_ws(a, chunk, &splits);
+    size_t need = mla_ws(a, chunk, &splits);
+    const int fit = ws ? plan_fit(ws_bytes, mla_split_bytes(a), stride_bound(a->max_seq_len, mla_tile_tokens(kernel), 0)) : 0;
+    const bool dev = mla_device_plan(a, kernel) && chunk > kPlanStaticChunk && fit >= splits;
+    if (dev) need = mla_ws(a, chunk, &splits, fit);
     if (!ws || ws_bytes < need)
         return fail(MUGEN_ATTN_E_WORKSPACE, "mla_decode: workspace of %zu bytes required, %zu given", need,
                     ws_bytes);
@@ -916,12 +977,13 @@ static int mla_decode_impl(const mugen_attn_mla_decode_args* a, void* ws, size_t
     p.R = a->q_len * a->n_heads;
     p.nrb = ceil_div(p.R, mla_rows_per_block(kernel));
     p.nq = ceil_div(p.R, 16);
-    const int64_t units = mla_units(a, chunk, p.nrb);
+    const int64_t units = dev ? std::min<int64_t>(kMlaBudget, (int64_t)a->batch * p.nrb * splits)
+                              : mla_units(a, chunk, p.nrb);
     // the kernels number the work units and the grid in 32 bits
     if (units > (int64_t)1 << 30)
         return fail(MUGEN_ATTN_E_UNSUPPORTED, "mla_decode: batch * splits * row blocks too large");
     p.units = (int)units;
-    p.chunk = chunk;
+    p.chunk = dev ? 0 : chunk;
     p.num_splits = splits;
     p.max_T = a->max_seq_len;
     p.seq_stride = a->seq_stride;
@@ -931,6 +993,7 @@ static int mla_decode_impl(const mugen_attn_mla_decode_args* a, void* ws, size_t
         const size_t sb = (size_t)a->batch * splits;
         p.ws_o = base;
         p.ws_ml = base + sb * (size_t)p.nq * 16 * 512 / 2;  // after the fp16 O blob
+        p.plan = reinterpret_cast<int*>(p.ws_ml + sb * (size_t)p.R * 2);
     }
     hipError_t e = launch_mla_decode(p, kernel, a->q_dtype, a->latent_dtype, a->out_dtype,
                                      static_cast<hipStream_t>(stream), timer);

@@ -255,6 +255,152 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v + dpp_xor<1>(v);
 }
 
+__device__ __forceinline__ int wave_sum_i32(int v) {
+    const auto r32 = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+    v = (int)r32[0] + (int)r32[1];
+    const auto r16 = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+    v = (int)r16[0] + (int)r16[1];
+    v += __float_as_int(dpp_xor<8>(__int_as_float(v)));
+    v += __float_as_int(dpp_xor<4>(__int_as_float(v)));
+    v += __float_as_int(dpp_xor<2>(__int_as_float(v)));
+    return v + __float_as_int(dpp_xor<1>(__int_as_float(v)));
+}
+// inclusive prefix sum over the wave's lanes: row shifts by 1, 2, 4, 8, then
+// lane 15 of each 16-lane row broadcast to the next row and lane 31 to the
+// upper half
+__device__ __forceinline__ int wave_scan_i32(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);
+    return v + __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+}
+
+// ceil(n / d) for 0 <= n < 2^23, 1 <= d, rd = 1.0f / d: the product is within
+// one of the quotient, the remainder tells which
+__device__ __forceinline__ int ceil_div_f(int n, int d, float rd) {
+    const int x = n + d - 1;
+    int q = (int)((float)x * rd);
+    const int r = x - q * d;
+    return r < 0 ? q - 1 : r >= d ? q + 1 : q;
+}
+
+// The context-split plan from the lengths on the device, for calls without
+// host lengths (captured decode steps: one plan made for max_seq_len would
+// leave most workgroups without work in a cache that is not full).  A chunk of
+// 32-token units, at least cmin, that cuts the longest sequence into at most
+// `cap` splits and whose work list -- mult items per split, count(j, c)
+// splits of sequence j at chunk c -- fits `budget` workgroups (B mult <=
+// budget / 2); every wave computes the same one.  units(j): 32-token units of
+// sequence j.  The kernels wait for it, so up to 8 sequences take one guess
+// (half a split's tokens lost per sequence) and else the closed bound sum mult /
+// (budget - B mult), which always fits (one sequence: a search cost 0.8 us of a
+// 7 us call), and more the smallest chunk to 1/16, searched from that guess.
+template <typename Units, typename Count>
+__device__ __forceinline__ int plan_chunk_device(int B, int mult, int budget, int cmin, int cap,
+                                                 Units units, Count count) {
+    const int lane = threadIdx.x & 63;
+    // an upper bound of ceil(n / d), at most one above it
+    auto div_up = [](int n, int d) {
+        return (int)((float)n * __builtin_amdgcn_rcpf((float)d) * (1.0f + 4e-6f)) + 1;
+    };
+    const float rcap = __builtin_amdgcn_rcpf((float)cap);
+    auto by_cap = [&](int mx) { return max(cmin, cap == 32 ? (mx + 31) >> 5 : ceil_div_f(mx, cap, rcap)); };
+    // the longest sequence cut evenly, where that still fits; else the bound
+    auto choose = [&](int sum, int mx, int c0, auto total) {
+        int c = max(c0, div_up(sum * mult, budget - B * mult / 2) - 1);
+        const int ns = ceil_div_f(mx, c, __builtin_amdgcn_rcpf((float)c));
+        c = max(c0, ceil_div_f(mx, ns, __builtin_amdgcn_rcpf((float)ns)));
+        if (total(c, __builtin_amdgcn_rcpf((float)c)) * mult > budget) c = max(c0, div_up(sum * mult, budget - B * mult));
+        return c;
+    };
+    // work lists that fit however the sequences are cut: the split cap alone
+    const bool fits = B * mult * cap <= budget;
+    if (B <= 4) {  // scalar loads, all at once (indices past B repeat the last sequence)
+        int u[4], sum = 0, mx = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            u[j] = units(min(j, B - 1));
+            mx = max(mx, u[j]);
+            sum += j < B ? u[j] : 0;
+        }
+        const int c = by_cap(mx);
+        if (fits || mx == 0) return 32 * c;
+        return 32 * __builtin_amdgcn_readfirstlane(choose(sum, mx, c, [&](int x, float rx) {
+                   int n = 0;
+#pragma unroll
+                   for (int j = 0; j < 4; j++)
+                       if (j < B) n += count(j, x, rx);
+                   return n;
+               }));
+    }
+    if (B <= 8) {
+        auto fold = [](int v, auto op) {
+            v = op(v, __float_as_int(dpp_xor<1>(__int_as_float(v))));
+            v = op(v, __float_as_int(dpp_xor<2>(__int_as_float(v))));
+            v = op(v, __float_as_int(dpp_xor<4>(__int_as_float(v))));
+            return __builtin_amdgcn_readfirstlane(v);
+        };
+        auto add = [](int a, int b) { return a + b; };
+        const int l = lane & 7, u = l < B ? units(l) : 0;
+        const int mx = fold(u, [](int a, int b) { return max(a, b); });
+        const int c = by_cap(mx);
+        if (fits || mx == 0) return 32 * c;
+        return 32 * __builtin_amdgcn_readfirstlane(
+                        choose(fold(u, add), mx, c, [&](int x, float rx) { return fold(l < B ? count(l, x, rx) : 0, add); }));
+    }
+    int sum = 0, mx = 0;
+    for (int j = lane; j < B; j += 64) {
+        const int u = units(j);
+        sum += u;
+        mx = max(mx, u);
+    }
+    sum = __builtin_amdgcn_readfirstlane(wave_sum_i32(sum));
+    mx = -__builtin_amdgcn_readfirstlane(wave_min_i32(-mx));
+    int c = __builtin_amdgcn_readfirstlane(
+        max(by_cap(mx), div_up(sum * mult, budget - B * mult / 2) - 1));
+    while (c < mx) {
+        const float rc = 1.0f / (float)c;
+        int n = 0;
+        for (int j = lane; j < B; j += 64) n += count(j, c, rc);
+        if (__builtin_amdgcn_readfirstlane(wave_sum_i32(n)) * mult <= budget) break;
+        c += max(1, c >> 4);
+    }
+    return c * 32;
+}
+
+// Work item -> sequence: sequence j has n(j) items, numbered in order; sets j
+// and the item's index in it, false past the last item.  Up to 4 sequences a
+// scalar loop, more a prefix sum over the lanes (32 sequences of 16 heads, MLA
+// decode: 28.4 -> 22.6 us against a loop over the batch)
+template <typename N>
+__device__ __forceinline__ bool find_sequence(int B, int item, N n, int& j, int& r) {
+    if (B <= 4) {
+        r = item;
+        for (j = 0; j < B; j++) {
+            const int c = n(j);
+            if (r < c) return true;
+            r -= c;
+        }
+        return false;
+    }
+    const int lane = threadIdx.x & 63;
+    for (int j0 = 0; j0 < B; j0 += 64) {
+        const int c = j0 + lane < B ? n(j0 + lane) : 0;
+        const int incl = wave_scan_i32(c);
+        const uint64_t past = __ballot(incl > item);
+        if (past) {
+            const int l = __builtin_ctzll(past);
+            j = j0 + l;
+            r = item - (__builtin_amdgcn_readlane(incl, l) - __builtin_amdgcn_readlane(c, l));
+            return true;
+        }
+        item -= __builtin_amdgcn_readlane(incl, 63);
+    }
+    return false;
+}
+
 // Split-K log-sum-exp weights for one output row: given the (m, l) pairs of
 // nact splits (m in log2 units, stride 2 floats apart by `ml_stride`),
 // writes f_s = 2^(m_s - M) to LDS and returns 1 / sum_s f_s l_s (0 when

@@ -70,15 +70,31 @@ __device__ __forceinline__ u32x4_t dequant_q4x8(uint32_t sm, uint32_t nib) {
 // one), or for the 4-bit store those of the Q4 tokens plus those of the f16
 // ring tokens (at least one)
 template <bool Q4>
-__device__ __forceinline__ int splits_of(const GqaDecodeParams& p, int j) {
+__device__ __forceinline__ int splits_of(const GqaDecodeParams& p, int j, int chunk) {
     const int Tj = clamp_len(p.seq_lens[j], p.max_T);
     if constexpr (Q4) {
         const int nqj = min(p.n_q4[j], max(Tj, 0));
-        const int n = (nqj + p.chunk - 1) / p.chunk + (max(Tj - nqj, 0) + p.chunk - 1) / p.chunk;
+        const int n = (nqj + chunk - 1) / chunk + (max(Tj - nqj, 0) + chunk - 1) / chunk;
         return n > 0 ? n : 1;
     } else {
-        return Tj > 0 ? (Tj + p.chunk - 1) / p.chunk : 1;
+        return Tj > 0 ? (Tj + chunk - 1) / chunk : 1;
     }
+}
+
+// the device plan of this call (plan_chunk_device)
+template <bool Q4>
+__device__ __forceinline__ int plan_gqa(const GqaDecodeParams& p) {
+    auto len = [&](int j) { return (clamp_len(p.seq_lens[j], p.max_T) + 31) >> 5; };
+    auto q4u = [&](int j) { return (clamp_len(min(p.n_q4[j], p.seq_lens[j]), p.max_T) + 31) >> 5; };
+    auto ring = [&](int j) {
+        const int T = clamp_len(p.seq_lens[j], p.max_T);
+        return (T - min(clamp_len(p.n_q4[j], p.max_T), T) + 31) >> 5;
+    };
+    return plan_chunk_device(
+        p.B, p.Hk, p.budget, 2, Q4 ? p.num_splits - 1 : p.num_splits, [&](int j) { return Q4 ? q4u(j) + ring(j) : len(j); },
+        [&](int j, int c, float rc) {
+            return max(1, Q4 ? ceil_div_f(q4u(j), c, rc) + ceil_div_f(ring(j), c, rc) : ceil_div_f(len(j), c, rc));
+        });
 }
 
 }  // namespace
@@ -108,23 +124,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1
     // 4-bit store: a kv head's 80-byte group run shares cache lines with its
     // neighbours', so the kv heads of one (sequence, split) -- consecutive
     // items -- go to one XCD (workgroups are dealt to the 8 XCDs round-robin
-    // by blockIdx): item = xcd * per_xcd + slot
-    const int item = (Q4 && p.per_xcd > 0) ? (int)(blockIdx.x % 8) * p.per_xcd + (int)(blockIdx.x / 8) : (int)blockIdx.x;
+    // by blockIdx): item = xcd * per_xcd + slot, per_xcd = ceil(items / 8)
+    int chunk = p.chunk;
     if constexpr (PF) {  // prompt mode: one split per (token, kv head)
+        const int item = (int)blockIdx.x;
         if (item < p.B * p.Hk) {
             b = item / p.Hk;
             kvh = item - b * p.Hk;
         }
-    } else
-    for (int j = 0, r = item; j < p.B; j++) {  // uniform scalar loop over the batch
-        const int nsj = splits_of<Q4>(p, j);
-        if (r < nsj * p.Hk) {
-            b = j;
+    } else {
+        if (chunk == 0) chunk = plan_gqa<Q4>(p);  // no host lengths: planned here
+        int item = (int)blockIdx.x;
+        if constexpr (Q4) {
+            int per_xcd = p.per_xcd;
+            if (p.chunk == 0) {
+                int n = 0;
+                for (int j = threadIdx.x & 63; j < p.B; j += 64) n += splits_of<Q4>(p, j, chunk);
+                per_xcd = (__builtin_amdgcn_readfirstlane(wave_sum_i32(n)) * p.Hk + 7) / 8;
+            }
+            if ((int)(blockIdx.x / 8) >= per_xcd) return;
+            item = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
+        }
+        int r;
+        if (find_sequence(p.B, item, [&](int j) { return splits_of<Q4>(p, j, chunk) * p.Hk; }, b, r)) {
             s = r / p.Hk;
             kvh = r - s * p.Hk;
-            break;
+        } else {
+            b = -1;
         }
-        r -= nsj * p.Hk;
     }
     if (b < 0) return;  // grid padding (sized from an upper bound)
     // a split past the workspace's stride (a device length above the host
@@ -137,10 +164,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1
     // [n_q4, T) are split separately, so a split -- and every 32-token block
     // of it -- holds one kind only (Q4 splits first)
     const int nq = Q4 ? min(p.n_q4[b], max(T, 0)) : 0;
-    const int nsq = Q4 ? (nq + p.chunk - 1) / p.chunk : 0;
+    const int nsq = Q4 ? (nq + chunk - 1) / chunk : 0;
     const bool q4_split = Q4 && s < nsq;
-    const int t_begin = q4_split || !Q4 ? s * p.chunk : nq + (s - nsq) * p.chunk;
-    const int t_end = min(t_begin + p.chunk, q4_split ? nq : T);
+    const int t_begin = q4_split || !Q4 ? s * chunk : nq + (s - nsq) * chunk;
+    const int t_end = min(t_begin + chunk, q4_split ? nq : T);
+    // item 0 leaves the plan to the merge (after the last read of the lengths:
+    // an earlier store would turn those into vector loads, +0.6 us)
+    if (!PF && p.chunk == 0 && blockIdx.x == 0 && threadIdx.x == 0) *p.plan = chunk;
     if (p.num_splits > 1 && t_begin >= t_end) return;  // empty split (T <= 0): the combine skips it
     MUGEN_TRACE(0);
     const int G = p.G;
@@ -475,8 +505,11 @@ __global__ __launch_bounds__(64) void gqa_decode_combine_kernel(GqaDecodeParams 
     const int h = blockIdx.x, b = blockIdx.y, d = blockIdx.z * 64 + threadIdx.x;
     MUGEN_TRACE(8);
     const int T = clamp_len(p.seq_lens[b], p.max_T);
-    const int nact = p.n_q4 ? min(p.num_splits, T > 0 ? splits_of<true>(p, b) : 0)
-                            : min(p.num_splits, (T + p.chunk - 1) / p.chunk);
+    // the plan; a few sequences' is formed again, which is faster than reading
+    // a line that another XCD just wrote (2 sequences: 7.8 -> 7.4 us a call)
+    const int chunk = p.chunk ? p.chunk : p.B > 4 ? *p.plan : p.n_q4 ? plan_gqa<true>(p) : plan_gqa<false>(p);
+    const int nact = p.n_q4 ? min(p.num_splits, T > 0 ? splits_of<true>(p, b, chunk) : 0)
+                            : min(p.num_splits, (T + chunk - 1) / chunk);
     const int64_t bh = (int64_t)b * p.H + h;
     const float* ml = p.ws_ml + bh * p.num_splits * 2;
     const float* os = p.ws_o + bh * p.num_splits * D + d;
@@ -540,7 +573,7 @@ __global__ __launch_bounds__(64) void gqa_decode_combine_kernel(GqaDecodeParams 
 
 template <int D, int DT, int OUT_DT, bool Q4 = false>
 static hipError_t launch_gqa_t(const GqaDecodeParams& p, int nwg, hipStream_t st, KernelTimer* timer) {
-    const int grid = (Q4 && p.per_xcd > 0) ? 8 * p.per_xcd : nwg;
+    const int grid = Q4 ? 8 * ((nwg + 7) / 8) : nwg;
     hipError_t e = (!Q4 && p.hd != D)
                        ? launch_k(timer, "gqa_decode", gqa_decode_kernel<D, DT, OUT_DT, false, true>, dim3(grid),
                                   dim3(256), st, p)

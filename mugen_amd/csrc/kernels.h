@@ -67,6 +67,10 @@ struct GqaDecodeParams {
     // split); it sees pf_start + b + 1 keys if pf_causal, else max_T
     int pf_start;
     int pf_causal;
+    // chunk 0: the kernel plans the chunk from the device lengths for at most
+    // `budget` items (plan_chunk_device) and leaves it in *plan for the merge
+    int* plan;
+    int budget;
 };
 
 // nwg: workgroups of the compact work list (exact, or an upper bound)
@@ -172,6 +176,9 @@ struct MlaParams {
     int max_T;             // device lengths are clamped to [0, max_T] (the cache's size)
     int64_t seq_stride;
     float scale_log2;
+    // chunk 0: planned by the kernel for at most `units` units, as in
+    // GqaDecodeParams
+    int* plan;
 };
 
 // every kernel reads a sequence's length through this clamp: a device value

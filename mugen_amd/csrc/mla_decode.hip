@@ -81,13 +81,20 @@ __device__ __forceinline__ int64_t blob_pair(const MlaParams& p, int b, int s, i
     return ((((int64_t)b * p.num_splits + s) * p.nq + q) * 16 + dp) * 64 + lane;
 }
 
+// the device plan of this call (plan_chunk_device)
+__device__ __forceinline__ int plan_mla(const MlaParams& p) {
+    auto len = [&](int j) { return (clamp_len(p.seq_lens[j], p.max_T) + 31) >> 5; };
+    return plan_chunk_device(p.B, p.nrb, p.units, 1, p.num_splits, len,
+                             [&](int j, int c, float rc) { return ceil_div_f(len(j), c, rc); });
+}
+
 // First 64-row block of a sequence of T tokens that sees a key of split s.
 // Query row r of a q_len-token step sees T - q_len + r / H + 1 keys, so
 // block rb (rows 64 rb .. 64 rb + 63) sees split s iff (64 rb + 63) / H >=
 // s chunk - T + q_len; the last block, whose last row sees all T keys, sees
 // every split.  Decode steps (q_len 1): every block sees every split.
-__device__ __forceinline__ int mla_rb_first(const MlaParams& p, int T, int s) {
-    const int x = s * p.chunk - T + p.q_len;
+__device__ __forceinline__ int mla_rb_first(const MlaParams& p, int T, int s, int chunk) {
+    const int x = s * chunk - T + p.q_len;
     return x <= 0 ? 0 : min((p.H * x) >> 6, p.nrb - 1);
 }
 
@@ -105,33 +112,34 @@ __device__ __forceinline__ int mla_rb_first(const MlaParams& p, int T, int s) {
 // groups than XCDs (a long prompt: many row blocks, few splits).  The grid
 // is sized from the host's unit count (exact with the length hint, an upper
 // bound without); surplus workgroups exit at once.
-__device__ __forceinline__ bool mla_map(const MlaParams& p, int& b, int& s, int& rb) {
+template <bool PLAN>
+__device__ __forceinline__ bool mla_map(const MlaParams& p, int& b, int& s, int& rb, int& chunk) {
     const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
+    chunk = p.chunk;
+    if constexpr (PLAN) chunk = plan_mla(p);  // no host lengths: planned here
     if (p.q_len == 1) {  // decode: every block of every split
+        auto splits = [&](int j) { return (clamp_len(p.seq_lens[j], p.max_T) + chunk - 1) / chunk; };
         int nact = 0;
-        for (int j = 0; j < p.B; j++) nact += (clamp_len(p.seq_lens[j], p.max_T) + p.chunk - 1) / p.chunk;  // uniform scalar loop
+        if (p.B <= 4) {
+            for (int j = 0; j < p.B; j++) nact += splits(j);  // uniform scalar loop
+        } else {
+            for (int j = threadIdx.x & 63; j < p.B; j += 64) nact += splits(j);
+            nact = __builtin_amdgcn_readfirstlane(wave_sum_i32(nact));
+        }
         const int units = nact * p.nrb;
         const int upx = (units + 7) / 8;
         const int unit = xcd * upx + slot;
         if (slot >= upx || unit >= units) return false;
         const int grp = unit / p.nrb;
         rb = unit - grp * p.nrb;
-        for (int j = 0, acc = 0; j < p.B; j++) {
-            const int nsj = (clamp_len(p.seq_lens[j], p.max_T) + p.chunk - 1) / p.chunk;
-            if (grp < acc + nsj) {
-                b = j;
-                s = grp - acc;
-                return s < p.num_splits;  // (a split past the partials' stride: nothing to write it to)
-            }
-            acc += nsj;
-        }
-        return false;
+        return find_sequence(p.B, grp, splits, b, s)
+               && s < p.num_splits;  // (a split past the partials' stride: nothing to write it to)
     }
     // causal multi-token step: the splits every block sees (s chunk <=
     // T - q_len) whole, then the last few from mla_rb_first on
     auto split_range = [&](int Tj, int& nsj, int& s0) {
-        nsj = (Tj + p.chunk - 1) / p.chunk;
-        s0 = min(nsj, Tj >= p.q_len ? (Tj - p.q_len) / p.chunk + 1 : 0);
+        nsj = (Tj + chunk - 1) / chunk;
+        s0 = min(nsj, Tj >= p.q_len ? (Tj - p.q_len) / chunk + 1 : 0);
     };
     int units = 0;  // uniform scalar loops
     for (int j = 0; j < p.B; j++) {
@@ -139,7 +147,7 @@ __device__ __forceinline__ bool mla_map(const MlaParams& p, int& b, int& s, int&
         int nsj, s0;
         split_range(Tj, nsj, s0);
         units += s0 * p.nrb;
-        for (int sj = s0; sj < nsj; sj++) units += p.nrb - mla_rb_first(p, Tj, sj);
+        for (int sj = s0; sj < nsj; sj++) units += p.nrb - mla_rb_first(p, Tj, sj, chunk);
     }
     const int upx = (units + 7) / 8;
     const int unit = xcd * upx + slot;
@@ -157,7 +165,7 @@ __device__ __forceinline__ bool mla_map(const MlaParams& p, int& b, int& s, int&
         }
         acc += s0 * p.nrb;
         for (int sj = s0; sj < nsj; sj++) {
-            const int first = mla_rb_first(p, Tj, sj);
+            const int first = mla_rb_first(p, Tj, sj, chunk);
             if (unit < acc + p.nrb - first) {
                 b = j;
                 s = sj;
@@ -174,7 +182,7 @@ __device__ __forceinline__ bool mla_map(const MlaParams& p, int& b, int& s, int&
 // workgroup = (64 query rows, context split, sequence), 4 waves of 16
 // rows, one wave per SIMD.  Each wave keeps the q of its rows in registers
 // (B operand of S^T = L . Q^T) and its 16 x 512 O accumulator.
-template <int QDT, int DT>
+template <int QDT, int DT, bool PLAN>
 __global__ __launch_bounds__(256) void mla_decode_kernel(MlaParams p) {
     constexpr int KS = kCD / 32;  // 18 k-steps over the 576 dims
     constexpr int NQ = (QDT == DT_F32) ? 2 : 1;
@@ -184,17 +192,21 @@ __global__ __launch_bounds__(256) void mla_decode_kernel(MlaParams p) {
     constexpr int DSTRIDE = NW * 1024;         // LDS bytes between a wave's DMA ops
     __shared__ __attribute__((aligned(1024))) char ring[kNBuf * kTileBytes];
 
-    int b, s, rb;
-    if (!mla_map(p, b, s, rb)) return;  // grid padding past the last active unit
+    int b, s, rb, chunk;
+    const bool live = mla_map<PLAN>(p, b, s, rb, chunk);
+    const int T = live ? clamp_len(p.seq_lens[b], p.max_T) : 0;
+    // the plan for the merge, after the last read of the lengths (an earlier
+    // store would turn those into vector loads)
+    if (PLAN && blockIdx.x == 0 && threadIdx.x == 0) *p.plan = chunk;
+    if (!live) return;  // grid padding past the last active unit
     MUGEN_TRACE(0);
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
     const int n = lane & 15, g = lane >> 4;
-    const int T = clamp_len(p.seq_lens[b], p.max_T);
-    const int t_begin = s * p.chunk;
-    const int t_end = min(t_begin + p.chunk, T);
+    const int t_begin = s * chunk;
+    const int t_end = min(t_begin + chunk, T);
     // tiles past the last visible token of the workgroup's last row (a
     // causal prompt's early rows) are not walked; a split that no row of
     // the workgroup sees stores an empty partial (m = -inf, l = 0, o = 0)
@@ -492,7 +504,7 @@ __global__ __launch_bounds__(256) void mla_decode_kernel(MlaParams p) {
 // S waves, one by the PV waves) and a double-buffered P.  One barrier per
 // tile: at barrier j the S waves have written P(j-1) and the PV waves have
 // finished tile j-2, whose slot then receives tile j+2.
-template <int QDT, int DT>
+template <int QDT, int DT, bool PLAN>
 __global__ __launch_bounds__(512) void mla_decode_ws_kernel(MlaParams p) {
     constexpr int KS = kCD / 32;          // 18 k-steps over the 576 dims
     // fp32 q: each S wave holds q as hi + lo 16-bit parts (RNE split) and
@@ -508,8 +520,13 @@ __global__ __launch_bounds__(512) void mla_decode_ws_kernel(MlaParams p) {
     __shared__ __attribute__((aligned(16))) float rs_alpha[2][64];  // per tile parity and row: O's re-base factor
     __shared__ __attribute__((aligned(16))) int rs_flag[2][4];  // per tile parity and S wave: any row re-based
 
-    int b, s, rb;
-    if (!mla_map(p, b, s, rb)) return;
+    int b, s, rb, chunk;
+    const bool live = mla_map<PLAN>(p, b, s, rb, chunk);
+    const int T = live ? clamp_len(p.seq_lens[b], p.max_T) : 0;
+    // the plan for the merge, after the last read of the lengths (an earlier
+    // store would turn those into vector loads)
+    if (PLAN && blockIdx.x == 0 && threadIdx.x == 0) *p.plan = chunk;
+    if (!live) return;
     MUGEN_TRACE(0);
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -517,9 +534,8 @@ __global__ __launch_bounds__(512) void mla_decode_ws_kernel(MlaParams p) {
     const bool s_wave = w < 4;
     const int wr = w & 3;  // S wave: row block; PV wave: column quarter
     const int n = lane & 15, g = lane >> 4;
-    const int T = clamp_len(p.seq_lens[b], p.max_T);
-    const int t_begin = s * p.chunk;
-    const int t_end = min(t_begin + p.chunk, T);
+    const int t_begin = s * chunk;
+    const int t_end = min(t_begin + chunk, T);
     const int row0 = rb * 64;  // first query row of the workgroup
     // tiles past the last visible token of the workgroup's last row (a
     // causal prompt's early rows) are not walked; a split that no row of
@@ -833,12 +849,13 @@ __global__ __launch_bounds__(64 * NW) void mla_decode_combine_kernel(MlaParams p
     const int tid = threadIdx.x, lane = tid & 63, dsub = tid >> 6;
     const int g = lane >> 4, n = lane & 15;
     const int T = clamp_len(p.seq_lens[b], p.max_T);
-    int nact = min(p.num_splits, (T + p.chunk - 1) / p.chunk);
+    const int chunk = p.chunk ? p.chunk : p.B > 4 ? *p.plan : plan_mla(p);  // (as gqa_decode_combine)
+    int nact = min(p.num_splits, (T + chunk - 1) / chunk);
     if (p.q_len > 1) {
         // the rows' 64-row block has units for the splits its last row sees
         // only (mla_map): the first ceil(visible / chunk)
         const int vis = T - p.q_len + min(qb / 4 * 64 + 63, p.R - 1) / p.H + 1;
-        nact = min(nact, (max(vis, 0) + p.chunk - 1) / p.chunk);
+        nact = min(nact, (max(vis, 0) + chunk - 1) / chunk);
     }
     const int64_t ml_st = (int64_t)p.R * 2;  // floats between splits of one row
     const float* ml0 = p.ws_ml + (int64_t)b * p.num_splits * p.R * 2;
@@ -959,12 +976,18 @@ __global__ __launch_bounds__(64 * NW) void mla_decode_combine_kernel(MlaParams p
 int mla_rows_per_block(int) { return 64; }
 int mla_tile_tokens(int) { return kTT; }
 
+template <int QDT, int DT, bool PLAN>
+static hipError_t launch_mla_main(const MlaParams& p, int kernel, hipStream_t st, KernelTimer* t) {
+    const int grid = 8 * ((p.units + 7) / 8);  // see mla_map
+    return kernel == 1
+               ? launch_k(t, "mla_decode", mla_decode_kernel<QDT, DT, PLAN>, dim3(grid), dim3(256), st, p)
+               : launch_k(t, "mla_decode", mla_decode_ws_kernel<QDT, DT, PLAN>, dim3(grid), dim3(512), st, p);
+}
+
 template <int QDT, int DT, int OUT_DT>
 static hipError_t launch_mla_t(const MlaParams& p, int kernel, hipStream_t st, KernelTimer* t) {
-    const int grid = 8 * ((p.units + 7) / 8);  // see mla_map
-    hipError_t e = kernel == 1
-                       ? launch_k(t, "mla_decode", mla_decode_kernel<QDT, DT>, dim3(grid), dim3(256), st, p)
-                       : launch_k(t, "mla_decode", mla_decode_ws_kernel<QDT, DT>, dim3(grid), dim3(512), st, p);
+    const hipError_t e = p.chunk == 0 ? launch_mla_main<QDT, DT, true>(p, kernel, st, t)
+                                      : launch_mla_main<QDT, DT, false>(p, kernel, st, t);
     if (e != hipSuccess) return e;
     // tiny merges (V2-Lite decode: one 16-row block of one sequence) spread
     // over more, smaller workgroups: 2 waves of 2 column blocks each (10.8 ->

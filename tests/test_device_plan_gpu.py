@@ -1,0 +1,106 @@
+"""Decode calls without host lengths: the kernels plan the context splits from
+the device lengths (one captured call serves every step of growing sequences).
+Against the oracle at batch sizes around a wave's 64 lanes, ragged and empty
+sequences and lengths around the split sizes, with the workspace between guard
+bands; and with a workspace of the static plan's size, which keeps that plan."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import mugen_amd
+from mugen_amd import _capi
+from mugen_amd import attention as A
+from tests import cases as C
+from tests.test_bounds_gpu import Guarded, guarded_ws
+
+pytestmark = pytest.mark.gpu
+
+
+def lens_of(B, hi, seed):
+    x = np.random.default_rng(seed).integers(0, hi + 1, B).astype(np.int32)
+    x[0] = hi
+    if B > 2:
+        x[1], x[B - 1] = 0, 1
+    return x
+
+
+@pytest.mark.parametrize("B,H,Hk,D,hi,cache", [
+    (1, 8, 8, 64, 700, 8192), (1, 7, 1, 128, 1, 6000), (1, 16, 16, 64, 6000, 6000), (4, 32, 32, 64, 777, 2048), (8, 16, 16, 64, 900, 1024), (5, 28, 4, 128, 1500, 4096),
+    (16, 16, 4, 128, 300, 1024), (64, 4, 4, 64, 400, 512), (65, 3, 1, 64, 500, 640), (127, 2, 2, 64, 130, 256),
+    (3, 8, 2, 256, 900, 2048), (2, 4, 2, 96, 64, 65),
+])
+def test_gqa_plan_on_device(device, B, H, Hk, D, hi, cache):
+    lens = lens_of(B, hi, B + hi)
+    c = C.gqa_decode_case(2100 + B, B, H, Hk, D, lens, max_T=cache, dtype=C.F16)
+    ref = C.gqa_decode_ref(c, nthreads=16)
+    q, k, v = (C.to_dev(c[x], C.F16, device) for x in ("qb", "kb", "vb"))
+    sl = torch.from_numpy(lens).to(device)
+    C.say(f"gqa_decode without host lengths B={B} Hk={Hk} D={D} lens<={hi} cache={cache}")
+    out = Guarded((B, H, D), torch.float32, device)
+    a = A.gqa_decode_args(q, k, v, sl, out.t, cache)
+    need = _capi.lib().mugen_attn_gqa_decode_workspace_size(ctypes.byref(a))
+    host = np.full(B, cache, np.int32)  # every sequence full: the plan for max_seq_len
+    a.seq_lens_host = host.ctypes.data
+    static = _capi.lib().mugen_attn_gqa_decode_workspace_size(ctypes.byref(a))
+    for size in (need, static):
+        ws = guarded_ws(size, device)
+        out.t.zero_()
+        mugen_amd.attention_decode(q, k, v, sl, cache, out=out.t, workspace=ws.t if size else None)
+        assert out.intact() and ws.intact(), "guard band overwritten"
+        C.assert_close(out.t.cpu().numpy(), ref, f"gqa plan on device, workspace {size}")
+
+
+@pytest.mark.parametrize("B,H,q_len,hi,cache", [(1, 16, 1, 1000, 8192), (8, 128, 1, 700, 2048), (3, 128, 5, 600, 1024),
+                                                (64, 16, 1, 90, 128), (65, 16, 1, 70, 96), (2, 16, 16, 333, 4096)])
+def test_mla_plan_on_device(device, B, H, q_len, hi, cache):
+    lens = np.maximum(lens_of(B, hi, B + hi), 0 if q_len == 1 else q_len).astype(np.int32)
+    c = C.mla_case(2200 + B, B, q_len, H, lens, max_T=cache, q_dtype=C.F32, lat_dtype=C.F16)
+    ref = C.mla_ref(c, nthreads=16)
+    q, lat = C.to_dev(c["q"], C.F32, device), C.to_dev(c["latb"], C.F16, device)
+    sl = torch.from_numpy(lens).to(device)
+    C.say(f"mla_decode without host lengths B={B} H={H} q_len={q_len} lens<={hi} cache={cache}")
+    out = Guarded((B, q_len, H, 512), torch.float32, device)
+    a = A.mla_args(q, lat, sl, out.t, cache, C.MLA_SCALE)
+    need = _capi.lib().mugen_attn_mla_decode_workspace_size(ctypes.byref(a))
+    host = np.full(B, cache, np.int32)
+    a.seq_lens_host = host.ctypes.data
+    static = _capi.lib().mugen_attn_mla_decode_workspace_size(ctypes.byref(a))
+    for size in (need, static):
+        ws = guarded_ws(size, device)
+        out.t.zero_()
+        mugen_amd.mla_attention(q, lat, sl, cache, scale=C.MLA_SCALE, out=out.t, workspace=ws.t)
+        assert out.intact() and ws.intact(), "guard band overwritten"
+        C.assert_close(out.t.cpu().numpy(), ref, f"mla plan on device, workspace {size}")
+
+
+@pytest.mark.parametrize("B,hi", [(1, 900), (5, 700), (66, 300)])
+def test_q4_plan_on_device(device, B, hi):
+    H, Hk, D, cache = 8, 2, 64, 1024
+    lens = lens_of(B, hi, B + hi)
+    kv = mugen_amd.KVCacheQ4(1, B, Hk, D, max_seq_len=cache, fp16_preserve_last=32, max_new=64, device=device)
+    g = torch.Generator(device=device).manual_seed(2300 + B)
+    k = torch.randn((B, hi, Hk * D), generator=g, device=device).half()
+    v = torch.randn((B, hi, Hk * D), generator=g, device=device).half()
+    for t in range(0, hi, 50):
+        kv.append(0, k[:, t:t + 50].contiguous(), v[:, t:t + 50].contiguous())
+        kv.advance()
+    q = torch.randn((B, H, D), generator=g, device=device).half()
+    # ragged lengths over the same store: the first len tokens, of which all
+    # but the newest 32 of the whole store are Q4
+    kv.seq_lens.copy_(torch.from_numpy(lens))
+    kv.n_q4.copy_(torch.from_numpy(np.minimum(lens, hi - 32).astype(np.int32)))
+    kv.seq_lens_host = lens.copy()
+    want = kv.attention_decode(0, q, out_dtype=torch.float32)
+    out = Guarded((B, H, D), torch.float32, device)
+    a = _capi.GqaDecodeQ4Args()
+    a.q, a.store, a.seq_lens, a.n_q4, a.out = q.data_ptr(), kv.store(0), kv.seq_lens.data_ptr(), kv.n_q4.data_ptr(), out.t.data_ptr()
+    a.batch, a.n_heads, a.n_kv_heads, a.head_dim, a.max_seq_len, a.out_dtype = B, H, Hk, D, cache, C.F32
+    L = _capi.lib()
+    need = L.mugen_attn_gqa_decode_q4_workspace_size(ctypes.byref(a))
+    ws = guarded_ws(need, device)
+    C.say(f"gqa_decode_q4 without host lengths B={B}")
+    _capi.check(L.mugen_attn_gqa_decode_q4(ctypes.byref(a), ctypes.c_void_p(ws.t.data_ptr()), need, A._stream(device)))
+    assert out.intact() and ws.intact(), "guard band overwritten"
+    C.assert_close(out.t.cpu().numpy(), want.cpu().numpy(), f"q4 plan on device B={B}")
