@@ -185,7 +185,31 @@ constexpr int kPlanSplitCap = 32, kGqaChunkMin = 64;
 // -> 10.0; B16 and B1 T4096 unchanged (their plans were ~32 splits).
 static int gqa_budget(const mugen_attn_gqa_decode_args* a) { return a->head_dim > 128 ? 256 : 512; }
 
-static int gqa_chunk(const mugen_attn_gqa_decode_args* a, int extra = 0) {
+// Large ragged batches.  Where the sequences alone (nearly) fill the round,
+// its chunk is far above the mean load of a workgroup and the longest
+// sequences run on when the others are done: 32 / 8 heads, 64 sequences of
+// 512..8191 tokens, one split each: 273 us, 4.3 TB/s.  Several rounds of
+// 1024-token items even that out: 236 us, 5.0 TB/s (2048 tokens 239, 512 239,
+// 256 260); 40 sequences 210 -> 177, 24 at 16 / 8 heads d256 240 -> 185, 64 at d64
+// 157 -> 129.  From 1.35 times the mean: equal lengths (363 us unsplit, 396 in
+// 1024s) and 48 sequences at 28 / 4 heads (1.23 times: 94.6 against 98.6) stay
+// in one round.  Needs the host lengths.
+constexpr int kGqaDeepChunk = 1024;
+static bool gqa_deep(const mugen_attn_gqa_decode_args* a, int chunk, int64_t budget) {
+    if (!a->seq_lens_host || chunk <= kGqaDeepChunk) return false;
+    int64_t sum = 0;
+    int longest = 0;
+    for (int b = 0; b < a->batch; b++) {
+        const int T = std::min(std::max(a->seq_lens_host[b], 0), a->max_seq_len);
+        sum += T;
+        longest = std::max(longest, T);
+    }
+    return (double)std::min(chunk, longest) * (double)budget > 1.35 * (double)sum * a->n_kv_heads;
+}
+
+// deep: false keeps the one-round plan (whose partials may fit a workspace
+// that the deep plan's do not)
+static int gqa_chunk(const mugen_attn_gqa_decode_args* a, int extra = 0, bool deep = true) {
     constexpr int q = 32, qmin = kGqaChunkMin, kSplitCap = kPlanSplitCap;
     const int maxT = a->max_seq_len > 0 ? a->max_seq_len : 1;
     if (a->num_splits > 0) return explicit_chunk(maxT, a->num_splits, q, kMaxSplits - 1);
@@ -211,7 +235,7 @@ static int gqa_chunk(const mugen_attn_gqa_decode_args* a, int extra = 0) {
         else lo = mid + q;
     }
     if (gqa_items(a, lo, extra) > budget) lo = hi;
-    return lo;
+    return deep && gqa_deep(a, lo, budget) ? std::max(kGqaDeepChunk, cmin) : lo;
 }
 
 static int gqa_validate(const mugen_attn_gqa_decode_args* a, bool ring_store = false) {
@@ -551,9 +575,10 @@ size_t mugen_attn_gqa_decode_q4_workspace_size(const mugen_attn_gqa_decode_q4_ar
 int mugen_attn_gqa_decode_q4(const mugen_attn_gqa_decode_q4_args* a, void* ws, size_t ws_bytes, void* stream) {
     if (int rc = gqa_q4_validate(a)) return rc;
     const mugen_attn_gqa_decode_args g = q4_as_gqa(a);
-    const int chunk = gqa_chunk(&g, 1);
+    int chunk = gqa_chunk(&g, 1);
     int splits = 2;
     size_t need = gqa_q4_ws(a, chunk, &splits);
+    if (ws_bytes < need) need = gqa_q4_ws(a, chunk = gqa_chunk(&g, 1, false), &splits);
     const int fit = ws ? plan_fit(ws_bytes, gqa_split_bytes(&g), stride_bound(a->max_seq_len, kGqaChunkMin, 1)) : 0;
     const bool dev = gqa_device_plan(&g, 1) && chunk > kPlanStaticChunk && fit >= splits;
     if (dev) need = gqa_q4_ws(a, chunk, &splits, fit);
@@ -613,9 +638,10 @@ size_t mugen_attn_gqa_decode_workspace_size(const mugen_attn_gqa_decode_args* a)
 int mugen_attn_gqa_decode(const mugen_attn_gqa_decode_args* a, void* ws, size_t ws_bytes, void* stream) {
     int rc = gqa_validate(a);
     if (rc) return rc;
-    const int chunk = gqa_chunk(a);
+    int chunk = gqa_chunk(a);
     int splits = 1;
     size_t need = gqa_ws(a, chunk, &splits);
+    if (!ws || ws_bytes < need) need = gqa_ws(a, chunk = gqa_chunk(a, 0, false), &splits);
     const int fit = ws ? plan_fit(ws_bytes, gqa_split_bytes(a), stride_bound(a->max_seq_len, kGqaChunkMin, 0)) : 0;
     const bool dev = gqa_device_plan(a, 0) && chunk > kPlanStaticChunk && fit > 1 && fit >= splits;
     if (dev) need = gqa_ws(a, chunk, &splits, fit);

@@ -104,3 +104,42 @@ def test_q4_plan_on_device(device, B, hi):
     _capi.check(L.mugen_attn_gqa_decode_q4(ctypes.byref(a), ctypes.c_void_p(ws.t.data_ptr()), need, A._stream(device)))
     assert out.intact() and ws.intact(), "guard band overwritten"
     C.assert_close(out.t.cpu().numpy(), want.cpu().numpy(), f"q4 plan on device B={B}")
+
+
+def test_gqa_deep_plan(device):
+    # a large ragged batch with host lengths: 1024-token items over several
+    # rounds; without their workspace the call keeps one split per sequence
+    B, H, Hk, D, cache = 64, 8, 8, 64, 2600
+    lens = lens_of(B, cache, 77)
+    c = C.gqa_decode_case(2400, B, H, Hk, D, lens, max_T=cache, dtype=C.F16)
+    ref = C.gqa_decode_ref(c, nthreads=16)
+    q, k, v = (C.to_dev(c[x], C.F16, device) for x in ("qb", "kb", "vb"))
+    sl = torch.from_numpy(lens).to(device)
+    C.say("gqa_decode deep plan")
+    for with_ws in (True, False):
+        out = Guarded((B, H, D), torch.float32, device)
+        a = A.gqa_decode_args(q, k, v, sl, out.t, cache)
+        a.seq_lens_host = lens.ctypes.data
+        L = _capi.lib()
+        need = L.mugen_attn_gqa_decode_workspace_size(ctypes.byref(a))
+        assert (need - 256) // (B * H * (4 * D + 8)) == 3  # 2600 tokens in 1024s
+        ws = guarded_ws(need, device)
+        _capi.check(L.mugen_attn_gqa_decode(ctypes.byref(a), ctypes.c_void_p(ws.t.data_ptr()) if with_ws else None,
+                                            need if with_ws else 0, A._stream(device)))
+        assert out.intact() and ws.intact(), "guard band overwritten"
+        C.assert_close(out.t.cpu().numpy(), ref, f"deep plan, workspace {with_ws}")
+
+
+def test_gqa_deep_plan_sizes():
+    # equal lengths stay in one round, unsplit (no workspace)
+    a = _capi.GqaDecodeArgs()
+    a.q = a.k_cache = a.v_cache = a.seq_lens = a.out = 0x1000
+    a.batch, a.n_heads, a.n_kv_heads, a.head_dim, a.max_seq_len = 64, 32, 8, 128, 8192
+    a.seq_stride, a.kv_dtype, a.out_dtype = 8192 * 8 * 128, C.F16, C.F16
+    size = _capi.lib().mugen_attn_gqa_decode_workspace_size
+    same = np.full(64, 8191, np.int32)
+    a.seq_lens_host = same.ctypes.data
+    assert size(ctypes.byref(a)) == 0
+    ragged = np.linspace(512, 8191, 64).astype(np.int32)
+    a.seq_lens_host = ragged.ctypes.data
+    assert (size(ctypes.byref(a)) - 256) // (64 * 32 * (4 * 128 + 8)) == 8
