@@ -21,6 +21,7 @@ from __future__ import annotations
 import ctypes
 import math
 
+import numpy as np
 import torch
 
 from . import _capi
@@ -39,15 +40,28 @@ def _ptr(t: torch.Tensor | None):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 
 
+# The wrappers run once per layer and step: a call of a few microseconds of GPU
+# work waits for them (no Stream object, no views made just for their sizes).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    if _raw_stream is None:  # a torch without device support
+        return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return ctypes.c_void_p(_raw_stream(device.index))
+
+
+def _per_sequence(t: torch.Tensor) -> int:
+    """Elements of one sequence's block of a [n_seq, ...] tensor."""
+    if t.shape[0] == 0:
+        raise IndexError("the cache holds no sequence")
+    return t.numel() // t.shape[0]
 
 
 def _host_lens(seq_lens_host):
     """int32 host array for the planner hint (or None)."""
     if seq_lens_host is None:
         return None
-    import numpy as np
     return np.ascontiguousarray(seq_lens_host, dtype=np.int32)
 
 
@@ -64,7 +78,7 @@ def _need_cuda(*ts: torch.Tensor):
 def gqa_decode_args(q, k_cache, v_cache, seq_lens, out, max_seq_len, scale=0.0, num_splits=0):
     B, H, D = q.shape
     Hk = k_cache.shape[-2]
-    seq_stride = k_cache[0].numel() if k_cache.dim() == 4 else 0
+    seq_stride = _per_sequence(k_cache) if k_cache.dim() == 4 else 0
     a = _capi.GqaDecodeArgs()
     a.q, a.k_cache, a.v_cache = q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr()
     a.seq_lens, a.out = seq_lens.data_ptr(), out.data_ptr()
@@ -164,7 +178,7 @@ def mla_args(q, latent, seq_lens, out, max_seq_len, scale, num_splits=0, kernel=
     a.q, a.latent, a.seq_lens, a.out = q.data_ptr(), latent.data_ptr(), seq_lens.data_ptr(), out.data_ptr()
     a.batch, a.q_len, a.n_heads, a.kv_rank, a.rope_dim = B, q_len, H, 512, C - 512
     a.max_seq_len, a.num_splits = int(max_seq_len), int(num_splits)
-    a.seq_stride = latent[0].numel()
+    a.seq_stride = _per_sequence(latent)
     a.scale = float(scale)
     a.q_dtype, a.latent_dtype, a.out_dtype = _dt(q.dtype), _dt(latent.dtype), _dt(out.dtype)
     a.kernel = int(kernel)
@@ -323,7 +337,7 @@ def _latent_args(kv_a, norm_w, positions, latent, rows_per_seq, eps, rope, max_s
     a.rows, a.rows_per_seq = rows, int(rows_per_seq)
     a.max_seq_len = int(latent.shape[1] if max_seq_len is None else max_seq_len)
     a.kv_rank, a.rope_dim, a.latent_dtype = 512, 64, _dt(latent.dtype)
-    a.seq_stride, a.eps, a.rope = latent[0].numel(), float(eps), _rope(rope)
+    a.seq_stride, a.eps, a.rope = _per_sequence(latent), float(eps), _rope(rope)
     if (rows + a.rows_per_seq - 1) // a.rows_per_seq > latent.shape[0]:
         raise ValueError("more sequences than latent has")
     return a
@@ -370,7 +384,7 @@ def kv_append(k_new: torch.Tensor, v_new: torch.Tensor, k_cache: torch.Tensor, v
         raise ValueError("k_new / v_new rows must match the caches' rows")
     a = _capi.KvAppendArgs()
     a.k_new, a.v_new, a.k_cache, a.v_cache = k_new.data_ptr(), v_new.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr()
-    a.seq_lens, a.seq_stride = seq_lens.data_ptr(), k_cache[0].numel()
+    a.seq_lens, a.seq_stride = seq_lens.data_ptr(), _per_sequence(k_cache)
     a.n_seq, a.n_new, a.row, a.max_seq_len = B, n_new, row, k_cache.shape[1]
     _capi.check(_capi.lib().mugen_attn_kv_append(ctypes.byref(a), _stream(k_new.device)))
 
