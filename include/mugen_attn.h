@@ -103,7 +103,8 @@ typedef struct mugen_attn_gqa_decode_args {
     int32_t kv_dtype;   /* mugen_attn_dtype */
     int32_t out_dtype;  /* mugen_attn_dtype */
     /* optional HOST copy of seq_lens (NULL allowed): lets the planner size
-     * the context splits for ragged batches.  It must equal the device
+     * the context splits for ragged batches; with NULL (and num_splits 0) the
+     * kernels plan them from the device lengths.  It must equal the device
      * lengths; a copy that is too short gives wrong results but never writes
      * outside the workspace.  The workspace size depends on it; a size asked
      * for without it (and num_splits 0) covers every host copy. */
@@ -320,7 +321,8 @@ typedef struct mugen_attn_mla_decode_args {
      * grid to exactly the active context splits, so every entry must be >=
      * the device value (normally equal; a larger value only costs idle
      * workgroups; a smaller one gives wrong results but never writes outside
-     * the workspace).  NULL sizes the grid for batch * max_seq_len.  The
+     * the workspace).  With NULL (and num_splits 0) the kernels plan the
+     * splits from the device lengths, where the workspace has room.  The
      * workspace size depends on it; a size asked for without it (and
      * num_splits 0) covers every host copy. */
     const int32_t* seq_lens_host;
