@@ -18,6 +18,7 @@
 #include <type_traits>
 
 #include "mugen_attn.h"
+#include "split_plan.h"
 
 namespace mugen_attn {
 
@@ -277,46 +278,20 @@ __device__ __forceinline__ int wave_scan_i32(int v) {
     return v + __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
 }
 
-// ceil(n / d) for 0 <= n < 2^23, 1 <= d, rd = 1.0f / d: the product is within
-// one of the quotient, the remainder tells which
-__device__ __forceinline__ int ceil_div_f(int n, int d, float rd) {
-    const int x = n + d - 1;
-    int q = (int)((float)x * rd);
-    const int r = x - q * d;
-    return r < 0 ? q - 1 : r >= d ? q + 1 : q;
-}
-
 // The context-split plan from the lengths on the device, for calls without
 // host lengths (captured decode steps: one plan made for max_seq_len would
 // leave most workgroups without work in a cache that is not full).  A chunk of
 // 32-token units, at least cmin, that cuts the longest sequence into at most
-// `cap` splits and whose work list -- mult items per split, count(j, c)
-// splits of sequence j at chunk c -- fits `budget` workgroups (B mult <=
-// budget / 2); every wave computes the same one.  units(j): 32-token units of
-// sequence j.  The kernels wait for it, so up to 8 sequences take one guess
-// (half a split's tokens lost per sequence) and else the closed bound sum mult /
-// (budget - B mult), which always fits (one sequence: a search cost 0.8 us of a
-// 7 us call), and more the smallest chunk to 1/16, searched from that guess.
-template <typename Units, typename Count>
+// `cap` splits (the store, KINDS 2: one more, see plan_few) and whose work list
+// -- mult items per split, count(j, c) splits of sequence j at chunk c -- fits
+// `budget` workgroups (the host sees to KINDS B mult <= budget); every wave
+// computes the same one.  units(j): 32-token units of sequence j.  The kernels
+// wait for it, so up to 8 sequences take one guess (plan_few), and more the
+// smallest chunk to 1/16, searched from that guess.
+template <int KINDS, typename Units, typename Count>
 __device__ __forceinline__ int plan_chunk_device(int B, int mult, int budget, int cmin, int cap,
                                                  Units units, Count count) {
     const int lane = threadIdx.x & 63;
-    // an upper bound of ceil(n / d), at most one above it
-    auto div_up = [](int n, int d) {
-        return (int)((float)n * __builtin_amdgcn_rcpf((float)d) * (1.0f + 4e-6f)) + 1;
-    };
-    const float rcap = __builtin_amdgcn_rcpf((float)cap);
-    auto by_cap = [&](int mx) { return max(cmin, cap == 32 ? (mx + 31) >> 5 : ceil_div_f(mx, cap, rcap)); };
-    // the longest sequence cut evenly, where that still fits; else the bound
-    auto choose = [&](int sum, int mx, int c0, auto total) {
-        int c = max(c0, div_up(sum * mult, budget - B * mult / 2) - 1);
-        const int ns = ceil_div_f(mx, c, __builtin_amdgcn_rcpf((float)c));
-        c = max(c0, ceil_div_f(mx, ns, __builtin_amdgcn_rcpf((float)ns)));
-        if (total(c, __builtin_amdgcn_rcpf((float)c)) * mult > budget) c = max(c0, div_up(sum * mult, budget - B * mult));
-        return c;
-    };
-    // work lists that fit however the sequences are cut: the split cap alone
-    const bool fits = B * mult * cap <= budget;
     if (B <= 4) {  // scalar loads, all at once (indices past B repeat the last sequence)
         int u[4], sum = 0, mx = 0;
 #pragma unroll
@@ -325,15 +300,14 @@ __device__ __forceinline__ int plan_chunk_device(int B, int mult, int budget, in
             mx = max(mx, u[j]);
             sum += j < B ? u[j] : 0;
         }
-        const int c = by_cap(mx);
-        if (fits || mx == 0) return 32 * c;
-        return 32 * __builtin_amdgcn_readfirstlane(choose(sum, mx, c, [&](int x, float rx) {
-                   int n = 0;
+        return 32 * __builtin_amdgcn_readfirstlane(plan_few<KINDS>(
+                        B, mult, budget, plan_by_cap(mx, cmin, cap), cap, sum, mx, [&](int x, float rx) {
+                            int n = 0;
 #pragma unroll
-                   for (int j = 0; j < 4; j++)
-                       if (j < B) n += count(j, x, rx);
-                   return n;
-               }));
+                            for (int j = 0; j < 4; j++)
+                                if (j < B) n += count(j, x, rx);
+                            return n;
+                        }));
     }
     if (B <= 8) {
         auto fold = [](int v, auto op) {
@@ -345,10 +319,9 @@ __device__ __forceinline__ int plan_chunk_device(int B, int mult, int budget, in
         auto add = [](int a, int b) { return a + b; };
         const int l = lane & 7, u = l < B ? units(l) : 0;
         const int mx = fold(u, [](int a, int b) { return max(a, b); });
-        const int c = by_cap(mx);
-        if (fits || mx == 0) return 32 * c;
         return 32 * __builtin_amdgcn_readfirstlane(
-                        choose(fold(u, add), mx, c, [&](int x, float rx) { return fold(l < B ? count(l, x, rx) : 0, add); }));
+                        plan_few<KINDS>(B, mult, budget, plan_by_cap(mx, cmin, cap), cap, fold(u, add), mx,
+                                        [&](int x, float rx) { return fold(l < B ? count(l, x, rx) : 0, add); }));
     }
     int sum = 0, mx = 0;
     for (int j = lane; j < B; j += 64) {
@@ -358,16 +331,13 @@ __device__ __forceinline__ int plan_chunk_device(int B, int mult, int budget, in
     }
     sum = __builtin_amdgcn_readfirstlane(wave_sum_i32(sum));
     mx = -__builtin_amdgcn_readfirstlane(wave_min_i32(-mx));
-    int c = __builtin_amdgcn_readfirstlane(
-        max(by_cap(mx), div_up(sum * mult, budget - B * mult / 2) - 1));
-    while (c < mx) {
-        const float rc = 1.0f / (float)c;
-        int n = 0;
-        for (int j = lane; j < B; j += 64) n += count(j, c, rc);
-        if (__builtin_amdgcn_readfirstlane(wave_sum_i32(n)) * mult <= budget) break;
-        c += max(1, c >> 4);
-    }
-    return c * 32;
+    const int c0 = __builtin_amdgcn_readfirstlane(
+        max(plan_by_cap(mx, cmin, cap), plan_div_up(sum * mult, budget - B * mult / 2) - 1));
+    return 32 * plan_grow(c0, mx, mult, budget, [&](int c, float rc) {
+               int n = 0;
+               for (int j = lane; j < B; j += 64) n += count(j, c, rc);
+               return __builtin_amdgcn_readfirstlane(wave_sum_i32(n));
+           });
 }
 
 // Work item -> sequence: sequence j has n(j) items, numbered in order; sets j

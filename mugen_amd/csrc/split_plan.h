@@ -1,0 +1,71 @@
+// split_plan.h -- arithmetic of the context-split plan made on the device
+// (plan_chunk_device, common.h): which chunk cuts the sequences of a batch into
+// a work list that the launch's workgroups cover.  Plain integer and float C++,
+// so that tests/cpp/split_plan_check.cpp runs the same code on the host.
+#pragma once
+
+#ifdef __HIPCC__
+#define MUGEN_PLAN_FN __device__ __forceinline__
+#else
+#define MUGEN_PLAN_FN inline
+#endif
+// 1 / x to one unit in the last place (v_rcp_f32)
+#ifndef MUGEN_PLAN_RCP
+#define MUGEN_PLAN_RCP(x) __builtin_amdgcn_rcpf(x)
+#endif
+
+namespace mugen_attn {
+
+MUGEN_PLAN_FN int plan_max(int a, int b) { return a > b ? a : b; }
+MUGEN_PLAN_FN float plan_rcp(int d) { return MUGEN_PLAN_RCP((float)d); }
+
+// ceil(n / d) for 0 <= n < 2^23, 1 <= d, rd = 1.0f / d to one ulp: the product
+// is within one of the quotient, the remainder tells which
+MUGEN_PLAN_FN int ceil_div_f(int n, int d, float rd) {
+    const int x = n + d - 1;
+    const int q = (int)((float)x * rd);
+    const int r = x - q * d;
+    return r < 0 ? q - 1 : r >= d ? q + 1 : q;
+}
+
+// an upper bound of ceil(n / d), at most one above it
+MUGEN_PLAN_FN int plan_div_up(int n, int d) { return (int)((float)n * plan_rcp(d) * (1.0f + 4e-6f)) + 1; }
+
+// the smallest chunk (in units, at least cmin) that cuts mx units into at most
+// cap splits
+MUGEN_PLAN_FN int plan_by_cap(int mx, int cmin, int cap) {
+    return plan_max(cmin, cap == 32 ? (mx + 31) >> 5 : ceil_div_f(mx, cap, plan_rcp(cap)));
+}
+
+// c, raised by a sixteenth at a time until its work list -- mult items for each
+// of the total(c, 1 / c) splits -- fits `budget`.  It ends at mx, where every
+// sequence is one split of each kind: the callers see to it that those fit
+template <typename Total>
+MUGEN_PLAN_FN int plan_grow(int c, int mx, int mult, int budget, Total total) {
+    while (c < mx && total(c, plan_rcp(c)) * mult > budget) c += plan_max(1, c >> 4);
+    return c;
+}
+
+// The plan of a few sequences from their units' sum and maximum mx.  KINDS: how
+// many runs of a sequence are split on their own (2: the 4-bit store's Q4 and
+// f16 tokens), each rounded up, so that a sequence has up to ceil(units / c) +
+// KINDS - 1 splits.  c0 = plan_by_cap.  KINDS B mult <= budget.
+template <int KINDS, typename Total>
+MUGEN_PLAN_FN int plan_few(int B, int mult, int budget, int c0, int cap, int sum, int mx, Total total) {
+    // work lists that fit however the sequences are cut: the split cap alone
+    if (B * mult * (cap + KINDS - 1) <= budget || mx == 0) return c0;
+    // one guess: half a split's tokens lost per rounding; the longest sequence
+    // cut evenly, where that still fits
+    int c = plan_max(c0, plan_div_up(sum * mult, budget - KINDS * B * mult / 2) - 1);
+    const int ns = ceil_div_f(mx, c, plan_rcp(c));
+    c = plan_max(c0, ceil_div_f(mx, ns, plan_rcp(ns)));
+    // the store: its two roundings leave no room for a closed bound where the
+    // batch fills half the round (budget = KINDS B mult), so the count decides
+    if (KINDS > 1) return plan_grow(c, mx, mult, budget, total);
+    // else the bound sum mult / (budget - B mult): one rounding per sequence, so
+    // it always fits (one sequence: a search cost 0.8 us of a 7 us call)
+    if (total(c, plan_rcp(c)) * mult > budget) c = plan_max(c0, plan_div_up(sum * mult, budget - B * mult));
+    return c;
+}
+
+}  // namespace mugen_attn

@@ -14,6 +14,7 @@ from mugen_amd import _capi
 from mugen_amd import attention as A
 from tests import cases as C
 from tests.test_bounds_gpu import Guarded, guarded_ws
+from tests.test_kv_q4_gpu import build_store, oracle_decode
 
 pytestmark = pytest.mark.gpu
 
@@ -24,6 +25,15 @@ def lens_of(B, hi, seed):
     if B > 2:
         x[1], x[B - 1] = 0, 1
     return x
+
+
+def planned(ws, size, per, bound):
+    """The chunk that the call left for its merge, after the partials of as many
+    splits (`per` bytes each, at most `bound`) as the workspace holds; None when
+    the call kept the static plan (the workspace was filled with 0xff)."""
+    fit = min((size - 512) // per, bound)
+    chunk = int(ws.t[fit * per:fit * per + 4].cpu().numpy().view(np.int32)[0])
+    return None if chunk == -1 else chunk
 
 
 @pytest.mark.parametrize("B,H,Hk,D,hi,cache", [
@@ -75,35 +85,48 @@ def test_mla_plan_on_device(device, B, H, q_len, hi, cache):
         C.assert_close(out.t.cpu().numpy(), ref, f"mla plan on device, workspace {size}")
 
 
-@pytest.mark.parametrize("B,hi", [(1, 900), (5, 700), (66, 300)])
-def test_q4_plan_on_device(device, B, hi):
-    H, Hk, D, cache = 8, 2, 64, 1024
-    lens = lens_of(B, hi, B + hi)
-    kv = mugen_amd.KVCacheQ4(1, B, Hk, D, max_seq_len=cache, fp16_preserve_last=32, max_new=64, device=device)
-    g = torch.Generator(device=device).manual_seed(2300 + B)
-    k = torch.randn((B, hi, Hk * D), generator=g, device=device).half()
-    v = torch.randn((B, hi, Hk * D), generator=g, device=device).half()
-    for t in range(0, hi, 50):
-        kv.append(0, k[:, t:t + 50].contiguous(), v[:, t:t + 50].contiguous())
-        kv.advance()
-    q = torch.randn((B, H, D), generator=g, device=device).half()
-    # ragged lengths over the same store: the first len tokens, of which all
-    # but the newest 32 of the whole store are Q4
-    kv.seq_lens.copy_(torch.from_numpy(lens))
-    kv.n_q4.copy_(torch.from_numpy(np.minimum(lens, hi - 32).astype(np.int32)))
-    kv.seq_lens_host = lens.copy()
-    want = kv.attention_decode(0, q, out_dtype=torch.float32)
+# the store rounds a sequence's Q4 and f16 tokens up to splits on their own: batches
+# whose work lists come closest to the launch's workgroups (equal lengths, half a
+# round of (sequence, kv head) pairs), each way to the plan.  A workspace of NaNs
+# shows a work item that nobody took
+@pytest.mark.parametrize("H,Hk,D,lens,keep,cache", [
+    (8, 8, 64, [4600, 5853, 3424, 4723, 5733, 5020, 4463, 3623], 256, 8192),
+    (8, 4, 64, [3054] * 4, 256, 4096),
+    (8, 8, 64, [5000] * 6, 256, 8192),
+    (8, 8, 64, [7168] * 2, 256, 8192),
+    (16, 8, 128, [2900], 100, 8192),
+    (2, 2, 256, [8000, 1, 0, 1024, 1024, 1024, 1024], 256, 8192),
+    (16, 16, 64, [1000 + 37 * i for i in range(16)], 200, 2048),
+    (4, 2, 64, [(131 * i) % 700 for i in range(66)], 32, 2048),
+])
+def test_q4_plan_on_device(device, H, Hk, D, lens, keep, cache):
+    B, T, ring = len(lens), max(lens), 256
+    nq = np.maximum(np.array(lens) - keep, 0).astype(np.int32)
+    rng = np.random.default_rng(2300 + B)
+    k, v, q = (rng.standard_normal(s, dtype=np.float32).astype(np.float16).view(np.uint16)
+               for s in ((B, T, Hk * D), (B, T, Hk * D), (B, H, D)))
+    store = build_store(k, v, lens, nq, ring, device)
+    for i in (0, 1):  # the Q4 rows as the first of a cache's
+        rows, store[i] = store[i], torch.zeros((B, cache, store[i].shape[2]), dtype=torch.uint8, device=device)
+        store[i][:, :T] = rows
+    qd, sl, nqd = C.to_dev(q, C.F16, device), torch.tensor(lens, dtype=torch.int32, device=device), torch.from_numpy(nq).to(device)
     out = Guarded((B, H, D), torch.float32, device)
     a = _capi.GqaDecodeQ4Args()
-    a.q, a.store, a.seq_lens, a.n_q4, a.out = q.data_ptr(), kv.store(0), kv.seq_lens.data_ptr(), kv.n_q4.data_ptr(), out.t.data_ptr()
+    a.store.q4_k, a.store.q4_v, a.store.ring_k, a.store.ring_v = [t.data_ptr() for t in store]
+    a.store.q4_seq_stride, a.store.ring_seq_stride = store[0][0].numel(), store[2][0].numel()
+    a.store.ring, a.store.fp16_preserve_last = ring, keep
+    a.q, a.seq_lens, a.n_q4, a.out = qd.data_ptr(), sl.data_ptr(), nqd.data_ptr(), out.t.data_ptr()
     a.batch, a.n_heads, a.n_kv_heads, a.head_dim, a.max_seq_len, a.out_dtype = B, H, Hk, D, cache, C.F32
     L = _capi.lib()
     need = L.mugen_attn_gqa_decode_q4_workspace_size(ctypes.byref(a))
     ws = guarded_ws(need, device)
-    C.say(f"gqa_decode_q4 without host lengths B={B}")
+    ws.t.fill_(255)
+    C.say(f"gqa_decode_q4 without host lengths B={B} Hk={Hk} D={D} lens<={T} cache={cache}")
     _capi.check(L.mugen_attn_gqa_decode_q4(ctypes.byref(a), ctypes.c_void_p(ws.t.data_ptr()), need, A._stream(device)))
     assert out.intact() and ws.intact(), "guard band overwritten"
-    C.assert_close(out.t.cpu().numpy(), want.cpu().numpy(), f"q4 plan on device B={B}")
+    chunk = planned(ws, need, B * H * (D * 4 + 8), min(32, -(-cache // 64)) + 1)
+    assert chunk is not None and chunk > 0 and chunk % 32 == 0, "the device plan is taken"
+    C.assert_close(out.t.cpu().numpy(), oracle_decode(q, k, v, lens, nq, H, Hk, D), f"q4 plan on device B={B}")
 
 
 def test_gqa_deep_plan(device):
