@@ -1003,12 +1003,7 @@ static int mla_decode_impl(const mugen_attn_mla_decode_args* a, void* ws, size_t
     p.R = a->q_len * a->n_heads;
     p.nrb = ceil_div(p.R, mla_rows_per_block(kernel));
     p.nq = ceil_div(p.R, 16);
-    // a planned decode step of a few sequences keeps a sixteenth of the round
-    // free: one tile more per split, fewer partials (V3 heads, B8 of 1024..8192
-    // tokens, 228 units instead of 252: fp32 q 28.8 -> 28.2 us on one machine, 26.9
-    // either way on another; 32 sequences 29.6 -> 30.2, so not there)
-    const int budget = a->q_len == 1 && p.nrb > 1 && a->batch <= 8 ? kMlaBudget * 15 / 16 : kMlaBudget;
-    const int64_t units = dev ? std::min<int64_t>(budget, (int64_t)a->batch * p.nrb * splits)
+    const int64_t units = dev ? std::min<int64_t>(kMlaBudget, (int64_t)a->batch * p.nrb * splits)
                               : mla_units(a, chunk, p.nrb);
     // the kernels number the work units and the grid in 32 bits
     if (units > (int64_t)1 << 30)

@@ -109,18 +109,18 @@ int main(int argc, char** argv) {
         store(std::vector<int>(6, 5000), 8, 512, 32, 256, "6 equal sequences x 8 kv heads");
         // every batch up to 64 that plans on the device, equal lengths and drawn
         // ones, every split cap that a workspace can leave
-        const int budgets[] = {256, 512, 240};
+        const int budgets[] = {256, 512, 256};  // GQA above head_dim 128 and up to it, MLA
         for (int bi = 0; bi < 3; bi++)
             for (int B = 1; B <= 64; B++)
                 for (int mult = 1; mult <= 32; mult++) {
-                    if (B * mult * 2 > (bi == 2 ? 256 : budgets[bi])) continue;
+                    if (B * mult * 2 > budgets[bi]) continue;
                     for (int T : {0, 1, 31, 33, 700, 3054, 4097, 7168, 8191, 32768}) {
                         if (bi < 2) store(std::vector<int>(B, T), mult, budgets[bi], 32, pick(0, 600), "equal");
                         check({1, mult, budgets[bi], bi == 2 ? 1 : 2, 32, bi < 2, std::vector<int>(B, T), {}}, "equal");
                     }
                 }
         for (int i = 0; i < draws; i++) {
-            const int bi = pick(0, 2), budget = budgets[bi], room = bi == 2 ? 128 : budget / 2;
+            const int bi = pick(0, 2), budget = budgets[bi], room = budget / 2;
             const int B = pick(0, 1) ? pick(1, 8) : pick(1, 64);
             const int mult = pick(1, std::max(1, room / B));
             if (B * mult > room) continue;
