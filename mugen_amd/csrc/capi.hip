@@ -20,6 +20,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "prefill_rules.h"
 
 namespace mugen_attn {
 
@@ -920,15 +921,8 @@ int mugen_attn_gqa_prefill(const mugen_attn_gqa_prefill_args* a, void* stream) {
         return hip_status(launch_gqa_prefill_wide(d, a->dtype, a->out_dtype, st, active_timer()),
                           "gqa_prefill launch");
     }
-    // below the flattened-row kernel's sizes: the warp-specialised kernel above
-    // head_dim 64 and for more than 4 heads per kv head (graph replays, us:
-    // Qwen2.5-7B shape N = 16 / 256 / 768 5.9 / 10.7 / 21.6 against 7.5 / 11.9 /
-    // 22.4 per-block, H32 Hk8 d128 N = 768 18.0 against 26.5; H16 Hk2 d64 N = 256
-    // 7.4 against 8.0); 4-head blocks at head_dim 64 from 1024 tokens (below, the
-    // per-block and short-prompt kernels lead: N = 512 7.7 against 9.2).
-    // args->kernel forces one
-    const bool ws_default =
-        a->head_dim > 64 || p.G > 4 || a->n_tokens >= 1024;
+    // below the flattened-row kernel's sizes (prefill_rules.h); args->kernel forces one
+    const bool ws_default = prefill_ws_default(a->n_tokens, p.G, a->head_dim);
     int kernel = ws_default ? MUGEN_ATTN_PREFILL_KERNEL_WS : MUGEN_ATTN_PREFILL_KERNEL_BLOCK;
     // prompts whose whole kv range fits on chip: the short-prompt kernel
     const bool short_fits = gqa_prefill_short_fits(p, padded_head_dim(a->head_dim));
