@@ -726,20 +726,6 @@ static bool gqa_prefill_v16_capable(const mugen_attn_gqa_prefill_args* a) {
     return a->head_dim <= 128 && a->dtype == DT_BF16;
 }
 
-// head_dim up to 128: the flattened-row kernel where its 128-row blocks make
-// enough workgroups (two share a CU, three at head_dim 64) that the longest
-// causal rows' chain does not set the time.  us, before (warp-specialised or
-// per-block) / flattened: 28 / 4 heads d128 448 workgroups (N = 2048) 42.3 / 47.9,
-// 672 90 / 82; 16 / 2 d128 512 77 / 94; 32 / 8 d128 512 52.5 / 50.7; d64 512 34.0 /
-// 37.0, 768 66 / 58; 14 / 2 d64 448 49 / 63, 656 105 / 98.  At 1 or 2 heads per kv head the 4-head blocks
-// of the warp-specialised kernel are at most half full: from 256 workgroups
-// (8 / 8 d128 129 / 83, 128 workgroups 40 / 44; 16 / 16 d64 256 43 / 34)
-static bool gqa_prefill_rows_default(const mugen_attn_gqa_prefill_args* a) {
-    const int G = a->n_heads / a->n_kv_heads;
-    const int64_t wgs = ((int64_t)a->n_tokens * G + 127) / 128 * a->n_kv_heads;
-    return wgs >= (G <= 2 ? 256 : G <= 4 && a->head_dim > 64 ? 512 : 640);
-}
-
 // head_dim above 128, keys not split: up to this many (token, kv head) pairs
 // (one round of workgroups) run one to a workgroup, whose four waves share
 // the pair's keys; past it the flattened-row kernel.  16 / 8 heads, us,
@@ -927,7 +913,8 @@ int mugen_attn_gqa_prefill(const mugen_attn_gqa_prefill_args* a, void* stream) {
     // prompts whose whole kv range fits on chip: the short-prompt kernel
     const bool short_fits = gqa_prefill_short_fits(p, padded_head_dim(a->head_dim));
     if (gqa_prefill_short_default(a)) kernel = MUGEN_ATTN_PREFILL_KERNEL_SHORT;
-    const bool rows = !a->kernel && kernel != MUGEN_ATTN_PREFILL_KERNEL_SHORT && gqa_prefill_rows_default(a);
+    const bool rows = !a->kernel && kernel != MUGEN_ATTN_PREFILL_KERNEL_SHORT &&
+                      prefill_rows_default(a->n_tokens, a->start_pos, a->causal, p.G, a->n_kv_heads, a->head_dim);
     if (a->kernel == MUGEN_ATTN_PREFILL_KERNEL_SHORT && !short_fits)
         return fail(MUGEN_ATTN_E_UNSUPPORTED,
                     "gqa_prefill: the short kernel serves head_dim 64, n_heads/n_kv_heads <= 4 and <= 512 keys");

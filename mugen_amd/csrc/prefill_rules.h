@@ -19,4 +19,42 @@ inline bool prefill_ws_default(int n_tokens, int G, int head_dim) {
     return head_dim > 64 || G > 4 || (n_tokens >= 1024 && n_tokens <= 4096);
 }
 
+// The flattened-row kernel where its 128-row blocks make enough workgroups (two
+// share a CU, three at head_dim 64) that the longest causal rows' chain does not
+// set the time, by how full the other kernels' head slots are: us, the faster
+// of those two / flattened.
+//  * head_dim above 64.  One or two heads per kv head (4-head blocks half full)
+//    256 workgroups: 8 / 8 heads 129 / 83, 16 / 8 47 / 44, 2 / 1 315 / 313, 128
+//    workgroups 40 / 44.  Up to 4: 512: 32 / 8 52.5 / 50.7, 8 / 2 191 / 182, 4 / 1
+//    375 / 360, 16 / 2 (8 heads each) 77 / 94.  More: 640: 28 / 4 heads 88 / 78,
+//    448 workgroups 42 / 48.  Where few kv heads make the blocks few and long, or
+//    all are equally long, 8-head slots full or one short need more: 8 / 1 640 243 /
+//    254, 768 333 / 324; after as many tokens 28 / 4 640 221 / 233, 768 321 / 296;
+//    32 / 4 640 185 / 187, 768 244 / 261 or 278 / 259 (where the other kernel's last
+//    round is full, or not), 1028 474 / 473, 1284 709 / 677.
+//  * head_dim 64.  One head per kv head 256: 16 / 16 43 / 34.  Two: more with fewer,
+//    longer chains, for which the per-block kernel's steps are shorter: 16 / 8 256
+//    27.3 / 34.0, 320 43.0 / 41.3; 8 / 4 320 77.2 / 77.4; 4 / 2 256 89 / 120, 384 182 /
+//    179; 2 / 1 384 334 / 356, 448 446 / 415; equally long 256: 16 / 8 after 8000 181 /
+//    150, 8 / 4 131 / 122, 2 / 1 448 / 477.  More: 640: 32 / 8 512 34 / 37, 768 66 / 58;
+//    14 / 2 448 49 / 63, 656 105 / 98; with full slots and one kv head 800: 4 / 1 640
+//    290 / 325, 750 388 / 399, 813 452 / 446; 8 / 1 640 158 / 166, 800 233 / 226.
+inline bool prefill_rows_default(int n_tokens, int start_pos, bool causal, int G, int n_kv_heads, int head_dim) {
+    const int64_t wgs = ((int64_t)n_tokens * G + 127) / 128 * n_kv_heads;
+    const bool level = !causal || start_pos >= n_tokens;  // blocks of about the same key count
+    int least = 640;
+    if (head_dim > 64) {
+        if (G <= 4) least = G <= 2 ? 256 : 512;
+        else if (G % 8 == 0) least = level ? 1088 : n_kv_heads <= 2 ? 768 : 640;
+        else if (G % 8 == 7 && level) least = 768;
+    } else if (G == 1) {
+        least = 256;
+    } else if (G == 2) {
+        least = level ? (n_kv_heads > 1 ? 256 : 320) : n_kv_heads >= 4 ? 320 : n_kv_heads > 1 ? 384 : 448;
+    } else if (!level && n_kv_heads == 1 && G % 4 == 0) {
+        least = 800;
+    }
+    return wgs >= least;
+}
+
 }  // namespace mugen_attn

@@ -63,10 +63,10 @@ def test_wide_rows_split(device, N, H, Hk, D, start, dtype):
 
 
 # head_dim up to 128: just past the workgroup counts where this kernel takes
-# over (256 at 1 or 2 heads per kv head, 512 up to 4 above head_dim 64, else 640),
-# with and without the fp16 copy of V.  The first rows, a stretch in the middle
+# over (256, 320, 512, 640: prefill_rows_default), with and without the fp16
+# copy of V.  The first rows, a stretch in the middle
 # and the last rows, through the oracle's start-offset form
-NARROW = [(2926, 28, 4, 128, 0), (1640, 40, 10, 96, 0), (1030, 32, 32, 128, 0), (1900, 33, 11, 64, 5),
+NARROW = [(2926, 28, 4, 128, 0), (1640, 40, 10, 96, 0), (1030, 32, 32, 128, 0), (1900, 33, 11, 64, 5), (2500, 33, 11, 64, 5),
           (3300, 16, 8, 64, 0), (860, 96, 16, 48, 3)]
 
 

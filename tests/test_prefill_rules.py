@@ -30,6 +30,24 @@ def choose(tmp_path_factory):
     (4097, 8, 2, 64, "block"), (9900, 8, 2, 64, "block"), (9000, 9, 3, 64, "block"), (20000, 4, 1, 64, "block"),
     (16000, 2, 1, 64, "block"),
     (64, 14, 2, 64, "ws"), (5000, 14, 2, 64, "ws"), (16, 28, 4, 128, "ws"), (2900, 28, 4, 128, "ws"), (700, 8, 2, 96, "ws"),
+    # from 128-row blocks enough on, the flattened-row kernel
+    (2926, 28, 4, 128, "rows"), (2048, 32, 8, 128, "rows"), (2047, 8, 8, 128, "ws"), (4096, 8, 8, 128, "rows"),
+    (1024, 32, 16, 128, "rows"), (2560, 32, 8, 64, "rows"), (5860, 14, 2, 64, "rows"), (1024, 32, 32, 64, "rows"),
+    # two heads per kv head at head_dim 64; full slots of one kv head
+    (2048, 16, 8, 64, "ws"), (2560, 16, 8, 64, "rows"), (8192, 4, 2, 64, "block"), (12288, 4, 2, 64, "rows"),
+    (24576, 2, 1, 64, "block"), (28672, 2, 1, 64, "rows"), (20500, 4, 1, 64, "block"), (26000, 4, 1, 64, "rows"),
+    (10300, 8, 1, 64, "ws"), (12800, 8, 1, 64, "rows"),
+    # 8 heads per kv head, full slots
+    (5180, 16, 2, 128, "ws"), (6144, 16, 2, 128, "rows"), (2620, 32, 4, 128, "rows"),
 ])
 def test_prompt_kernel(choose, N, H, Hk, D, kernel):
-    assert choose(N, H, Hk, D) == kernel
+    assert choose(N, 0, 1, H, Hk, D) == kernel
+
+
+# blocks of about the same key count: after a long context, or not causal
+@pytest.mark.parametrize("N,H,Hk,D,kernel", [
+    (2933, 28, 4, 128, "ws"), (3518, 28, 4, 128, "rows"), (2568, 32, 4, 128, "ws"), (3072, 32, 4, 128, "ws"), (4400, 32, 4, 128, "rows"),
+    (2048, 16, 8, 64, "rows"), (16384, 2, 1, 64, "block"), (20500, 4, 1, 64, "rows"), (3421, 24, 4, 128, "rows"), (2926, 28, 4, 64, "rows"),
+])
+def test_level_chunk_kernel(choose, N, H, Hk, D, kernel):
+    assert choose(N, N, 1, H, Hk, D) == kernel and choose(N, 0, 0, H, Hk, D) == kernel
