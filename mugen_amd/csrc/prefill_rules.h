@@ -40,6 +40,7 @@ inline bool prefill_ws_default(int n_tokens, int G, int head_dim) {
 //    14 / 2 448 49 / 63, 656 105 / 98; with full slots and one kv head 800: 4 / 1 640
 //    290 / 325, 750 388 / 399, 813 452 / 446; 8 / 1 640 158 / 166, 800 233 / 226.
 inline bool prefill_rows_default(int n_tokens, int start_pos, bool causal, int G, int n_kv_heads, int head_dim) {
+    if ((int64_t)n_tokens * G > INT32_MAX - 127) return false;  // the kernel numbers the rows in 32 bits
     const int64_t wgs = ((int64_t)n_tokens * G + 127) / 128 * n_kv_heads;
     const bool level = !causal || start_pos >= n_tokens;  // blocks of about the same key count
     int least = 640;

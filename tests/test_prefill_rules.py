@@ -51,3 +51,8 @@ def test_prompt_kernel(choose, N, H, Hk, D, kernel):
 ])
 def test_level_chunk_kernel(choose, N, H, Hk, D, kernel):
     assert choose(N, N, 1, H, Hk, D) == kernel and choose(N, 0, 0, H, Hk, D) == kernel
+
+
+def test_row_numbers_fit_32_bits(choose):
+    # 2^31 rows of a kv head: the kernel's row numbers would overflow
+    assert choose(2**27 - 8, 0, 0, 16, 1, 8) == "rows" and choose(2**27, 0, 0, 16, 1, 8) == "ws"
