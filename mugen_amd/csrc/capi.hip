@@ -781,7 +781,7 @@ static PrefillSplit prefill_split_plan(const mugen_attn_gqa_prefill_args* a, int
     r.kchunk = kchunk;
     // sized for `want` ranges (ks <= want): want never falls as the key
     // range grows, so the size at the longest range covers every shorter one
-    r.bytes = (size_t)a->n_tokens * a->n_heads * want * (part + 2 * sizeof(float)) + 512;
+    r.bytes = prefill_split_bytes((size_t)a->n_tokens * a->n_heads * want, part);
     return r;
 }
 
@@ -873,7 +873,7 @@ int mugen_attn_gqa_prefill(const mugen_attn_gqa_prefill_args* a, void* stream) {
             p.ksplit = split.ksplit;
             p.kchunk = split.kchunk;
             p.ws_ml = align256(a->workspace);
-            p.ws_o = reinterpret_cast<uint16_t*>(p.ws_ml + (size_t)a->n_tokens * a->n_heads * split.ksplit * 2);
+            p.ws_o = reinterpret_cast<uint16_t*>(p.ws_ml + prefill_partials_at((size_t)a->n_tokens * a->n_heads * split.ksplit));
         }
         if (p.ksplit > 1 || (int64_t)a->n_tokens * a->n_kv_heads > kPrefillWideItems) {
             hipError_t e = launch_gqa_prefill_rows(p, a->n_kv_heads, a->dtype, a->out_dtype, st, active_timer());
@@ -929,7 +929,7 @@ int mugen_attn_gqa_prefill(const mugen_attn_gqa_prefill_args* a, void* stream) {
         p.ksplit = split.ksplit;
         p.kchunk = split.kchunk;
         p.ws_ml = align256(static_cast<char*>(a->workspace) + v16_bytes);
-        p.ws_o = reinterpret_cast<uint16_t*>(p.ws_ml + (size_t)a->n_tokens * a->n_heads * split.ksplit * 2);
+        p.ws_o = reinterpret_cast<uint16_t*>(p.ws_ml + prefill_partials_at((size_t)a->n_tokens * a->n_heads * split.ksplit));
     }
     if (kernel != MUGEN_ATTN_PREFILL_KERNEL_SHORT && v16_bytes && a->workspace && a->workspace_bytes >= v16_bytes) {
         // V -> fp16 once for the whole call (the kernels then skip their

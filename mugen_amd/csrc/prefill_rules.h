@@ -1,7 +1,8 @@
-// prefill_rules.h -- which prefill kernel takes a prompt at head_dim up to 128.
-// Plain integer C++, so that tests/cpp/prefill_rules_check.cpp prints the same
-// choices on the host.
+// prefill_rules.h -- which prefill kernel takes a prompt at head_dim up to 128,
+// and where a split call's partials lie.  Plain integer C++, so that
+// tests/cpp/prefill_rules_check.cpp prints the same on the host.
 #pragma once
+#include <cstddef>
 #include <cstdint>
 
 namespace mugen_attn {
@@ -57,5 +58,12 @@ inline bool prefill_rows_default(int n_tokens, int start_pos, bool causal, int G
     }
     return wgs >= least;
 }
+
+// Key splits: floats from the (max, sum) pairs, at a 256-byte boundary of the
+// workspace, to the partials, which are read and written 16 bytes at a time: the
+// pairs of an odd number of (row, split) slots end between two such words
+inline size_t prefill_partials_at(size_t slots) { return (slots * 2 + 63) / 64 * 64; }
+// bytes for that many slots of `part` bytes, with both roundings
+inline size_t prefill_split_bytes(size_t slots, size_t part) { return slots * (part + 2 * sizeof(float)) + 512; }
 
 }  // namespace mugen_attn

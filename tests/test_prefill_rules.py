@@ -18,8 +18,8 @@ def choose(tmp_path_factory):
     subprocess.run([cxx, "-std=c++17", "-O1", "-I", os.path.join(ROOT, "mugen_amd", "csrc"),
                     os.path.join(ROOT, "tests", "cpp", "prefill_rules_check.cpp"), "-o", exe], check=True)
 
-    def run(*shape):
-        return subprocess.run([exe], input=" ".join(map(str, shape)) + "\n", check=True, capture_output=True,
+    def run(*shape, args=()):
+        return subprocess.run([exe, *args], input=" ".join(map(str, shape)) + "\n", check=True, capture_output=True,
                               text=True).stdout.strip()
     return run
 
@@ -56,3 +56,12 @@ def test_level_chunk_kernel(choose, N, H, Hk, D, kernel):
 def test_row_numbers_fit_32_bits(choose):
     # 2^31 rows of a kv head: the kernel's row numbers would overflow
     assert choose(2**27 - 8, 0, 0, 16, 1, 8) == "rows" and choose(2**27, 0, 0, 16, 1, 8) == "ws"
+
+
+@pytest.mark.parametrize("slots", [1, 7, 8, 31, 33, 255, 3 * 17 * 5, 100 * 16 * 8])
+@pytest.mark.parametrize("part", [2 * 8, 2 * 128, 4 * 136, 4 * 256])
+def test_split_partials_are_aligned(choose, slots, part):
+    # one token, one head, 7 key ranges: the pairs end 56 bytes past the boundary
+    at, size = map(int, choose(slots, part, args=("partials",)).split())
+    assert at % 16 == 0 and at >= 8 * slots
+    assert 255 + at + slots * part <= size, "the workspace covers both roundings"
