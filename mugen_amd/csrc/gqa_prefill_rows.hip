@@ -382,7 +382,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1
     }
     // tile j of slot u: S(j + 1) runs ahead into sn while the softmax of s
     // and the PV product of tile j - 1 are under way
-    auto step = [&](int j, f32x16_t& s, f32x16_t& sn) {
+    auto step = [&](int j, f32x16_t& s, f32x16_t& sn, bool first) {
         const int u = slot, un = u == NSLOT - 1 ? 0 : u + 1, up = u == 0 ? NSLOT - 1 : u - 1;
         slot = un;
         // V(j) and K(j + 1) landed (VCVT: and V(j + 1), whose conversion is due
@@ -401,7 +401,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1
             if (VCVT && left > 0) cv_write(un);
             return;
         }
-        if (__builtin_expect(j > 0 && j >= jmask, 0)) mask(s, k_beg + j * TK);
+        if (!first && __builtin_expect(j >= jmask, 0)) mask(s, k_beg + j * TK);
         float nm = m_run == kNegInf ? 0.f : -m_run;
         addr_k(un);
         addr_v(u);
@@ -441,7 +441,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1
         // re-base only when a lane's weights sum past kClampW (every weight
         // >= 0, so any weight past it shows).  A row without a visible key
         // in the first tile sees no later key
-        if (__builtin_expect(j > 0 && __any(!(ps <= kClampW)), 0)) {
+        if (!first && __builtin_expect(__any(!(ps <= kClampW)), 0)) {
             float mt = kNegInf;
 #pragma unroll
             for (int i = 0; i < 16; i++) mt = fmaxf(mt, fmaf(s[i], p.scale_log2, nm));
@@ -463,11 +463,39 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1
         l_part += ps;
 #pragma unroll
         for (int m = 0; m < 2; m++) split_p<PDT, NP>(x + 8 * m, pf[m]);
+        // the first tile: what rounding took off its weights, through the same
+        // V^T.  Rows of few keys have the largest outputs, and most of their keys
+        // here; the per-pair kernel's four reference weights of exactly 1 a row
+        // (here one) had a smaller error without it.  Against 64 bits, f16, 16 / 8
+        // heads d256, per pair / without / with: N = 150 2.34 / 2.43 / 2.16e-4, 1021
+        // 2.50 / 2.60 / 2.43e-4, 700 after 1500 2.907 / 2.910 / 2.891e-4; 28 / 4 heads
+        // d128 N = 3072, warp-specialised / without / with 2.63 / 2.65 / 2.51e-4
+        if (NP == 1 && first) {
+#pragma unroll
+            for (int m = 0; m < 2; m++) {
+                u32x4_t hl[2];
+                split_p<PDT, 2>(x + 8 * m, hl);
+#pragma unroll
+                for (int d = 0; d < DB; d++) o[d] = mfma32x32x16<PDT>(vf[m][d], hl[1], o[d]);
+            }
+        }
         if (VCVT && left > 0) cv_write(un);
     };
-    for (int j = 0; j < nt; j += 2) {
-        step(j, s0, s1);
-        if (j + 1 < nt) step(j + 1, s1, s0);
+    // the first tile on its own: no mask or re-base to test for, and the loop
+    // without its extra product (in the loop: 472 -> 475 us at 28 / 4 heads d128 N =
+    // 8192).  Padded heads above 128 keep it in the loop, whose schedule suffers from
+    // the copy (16 / 8 heads d192 N = 2048 78 against 84 us)
+    if constexpr (PAD && D > 128) {
+        for (int j = 0; j < nt; j += 2) {
+            step(j, s0, s1, j == 0);
+            if (j + 1 < nt) step(j + 1, s1, s0, false);
+        }
+    } else {
+        if (nt > 0) step(0, s0, s1, true);
+        for (int j = 1; j < nt; j += 2) {
+            step(j, s1, s0, false);
+            if (j + 1 < nt) step(j + 1, s0, s1, false);
+        }
     }
     if (nw > 0) pv();
 

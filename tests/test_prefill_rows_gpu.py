@@ -109,3 +109,43 @@ def test_rows_climbing_scores(device, N, H, Hk, D, dtype):
     c["q"], c["qb"] = C.O.round_to(q, dtype)
     c["k"], c["kb"] = C.O.round_to(k, dtype)
     check(c, device, f"climbing scores, head_dim {D}")
+
+
+def exact(q, k, v):
+    """Causal attention over a prompt in 64 bits, head by head."""
+    N, H, D = q.shape
+    G = H // k.shape[1]
+    hidden = torch.ones(N, N, dtype=torch.bool, device=q.device).triu(1)
+    out = torch.empty(N, H, D, dtype=torch.float64, device=q.device)
+    for h in range(H):
+        s = (q[:, h].double() @ k[:, h // G].double().T.contiguous()) / D ** 0.5
+        out[:, h] = torch.softmax(s.masked_fill(hidden, float("-inf")), 1) @ v[:, h // G].double()
+    return out
+
+
+@pytest.mark.parametrize("N,H,Hk,D", [(150, 16, 8, 256), (300, 16, 8, 256), (300, 16, 4, 192)])
+def test_rounding_of_the_weights(device, N, H, Hk, D):
+    # f16 weights, f32 output.  Their rounding leaves 2^-11 / sqrt(3) x 0.72 (log-
+    # uniform significands) = 2.0e-4 of the norm of sum p v, less what weights of
+    # exactly 1 save: 1.35e-4 in prompts of a few hundred tokens with a reference
+    # weight in each of four waves, 1.52e-4 with one.  The first tile's weights as
+    # two terms: 1.1e-4
+    g = torch.Generator(device=device).manual_seed(1700 + N)
+    q, k, v = (torch.randn(s, generator=g, device=device).half() for s in ((N, H, D), (N, Hk, D), (N, Hk, D)))
+    C.say(f"prefill rows, error against 64 bits N={N} D={D}")
+    ref = exact(q, k, v)
+    err = (mugen_amd.flash_prefill_attention(q, k, v, out_dtype=torch.float32).double() - ref).norm() / ref.norm()
+    assert err.item() < 1.35e-4
+
+
+def test_rounding_against_the_other_kernel(device):
+    # 7 heads per kv head: the warp-specialised kernel's reference is the largest
+    # of 64 scores, this kernel's of 32
+    N, H, Hk, D = 2926, 28, 4, 128
+    g = torch.Generator(device=device).manual_seed(1800)
+    q, k, v = (torch.randn(s, generator=g, device=device).half() for s in ((N, H, D), (N, Hk, D), (N, Hk, D)))
+    C.say("prefill rows and warp-specialised, error against 64 bits")
+    ref = exact(q, k, v)
+    err = [(mugen_amd.flash_prefill_attention(q, k, v, out_dtype=torch.float32, kernel=kernel).double() - ref).norm().item()
+           for kernel in (0, _capi.PREFILL_KERNEL_WS)]
+    assert err[0] <= err[1], err
