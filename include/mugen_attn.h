@@ -214,12 +214,15 @@ int mugen_attn_gqa_decode_q4(const mugen_attn_gqa_decode_q4_args* args, void* wo
  * Supported: head_dim a multiple of 8 up to 256 (as gqa_decode; above 128
  * only kernel 0 is accepted);
  * n_heads / n_kv_heads in [1, 16] (more
- * than 8 runs on the warp-specialised kernel; forcing the per-block kernel
- * there is refused); dtype F16 or BF16 for q/k/v; out_dtype F16/BF16/F32.
+ * than 8: forcing the per-block kernel is refused); dtype F16 or BF16 for q/k/v; out_dtype F16/BF16/F32.
  * With BF16 inputs the kernels may compute P.V in fp16 (V converted on
  * chip, exact inside the f16 range), so BF16 V values must lie
  * within +-65504 -- the range of the reference's f16 cache; V magnitudes
- * below 6.1e-5 keep an absolute precision of 2^-25.  The optional
+ * below 6.1e-5 keep an absolute precision of 2^-25.
+ * Infinities and NaNs in V: above head_dim 128 a token's result depends on the
+ * keys it attends to only.  Up to 128 a V row that is not finite also reaches
+ * earlier tokens of the same query block (as a weight of 0 times it), up to 31
+ * positions before it; finite caches are not concerned.  The optional
  * workspace (below) holds an fp16 copy of BF16 V for long prompts, and the
  * partials of split key ranges for short chunks over a long context.
  */

@@ -68,6 +68,53 @@ __device__ __forceinline__ f32x16_t mfma32x32x16(u32x4_t a, u32x4_t b, f32x16_t 
                                                       c, 0, 0, 0);
 }
 
+// One row without matrix products, over keys [k, end): a lane's dot product per
+// key, the weights handed round, each lane its output columns.  Nothing of a key
+// past `end` is read.  (m, l) as the rows of the main loop
+template <int D, int DT>
+__device__ __forceinline__ void row_by_hand(const GqaPrefillParams& p, const uint16_t* q, const uint16_t* kb,
+                                            const uint16_t* vb, int hd, int k, int end, float (&o)[D / 64], float& m,
+                                            float& l) {
+    const int lane = threadIdx.x & 63;
+    m = kNegInf;
+    l = 0.f;
+#pragma unroll
+    for (int c = 0; c < D / 64; c++) o[c] = 0.f;
+#pragma unroll 1
+    for (; k < end; k += 64) {
+        float s = kNegInf;
+        if (k + lane < end) {
+            const uint16_t* kr = kb + (int64_t)(k + lane) * p.row_stride;
+            s = 0.f;
+#pragma unroll 1
+            for (int c = 0; c < hd; c += 8) {
+                const u32x4_t x = load16(q + c), y = load16(kr + c);
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    s += lo_f32<DT>(x[e]) * lo_f32<DT>(y[e]) + hi_f32<DT>(x[e]) * hi_f32<DT>(y[e]);
+            }
+            s *= p.scale_log2;
+        }
+        const float mn = fmaxf(m, wave_max(s)), ref = mn == kNegInf ? 0.f : mn;
+        const float alpha = m == kNegInf ? 0.f : fast_exp2(m - ref);
+        const float w = fast_exp2(s - ref);
+        m = mn;
+        l = l * alpha + w;
+#pragma unroll
+        for (int c = 0; c < D / 64; c++) o[c] *= alpha;
+        const int n = min(64, end - k);
+#pragma unroll 1
+        for (int i = 0; i < n; i++) {
+            const float wi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), i));
+            const uint16_t* vr = vb + (int64_t)(k + i) * p.row_stride;
+#pragma unroll
+            for (int c = 0; c < D / 64; c++)
+                if (lane + 64 * c < hd) o[c] += wi * to_f32<DT>(vr[lane + 64 * c]);
+        }
+    }
+    l = wave_sum(l);
+}
+
 // 16-byte chunk c of K (and q) tile row r is stored at chunk c ^ rk_swz(r).
 // LDS has 64 banks x 4 B: a phase of a ds_read_b128 covers 16 lanes whose
 // rows differ in bits 0, 1, 3, 4 (lane quads of equal parity), and a row is
@@ -499,6 +546,51 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1
     }
     if (nw > 0) pv();
 
+    // partials: fp16 up to head_dim 128 (a convex combination of V rows, inside
+    // V's +-65504), fp32 above
+    constexpr int SDT = SPLIT ? (D > 128 ? DT_F32 : DT_F16) : OUT_DT;
+    // A key that a row does not see has weight 0 in the wave's tiles from mask_from
+    // on, and 0 x an infinity or a NaN of its V is a NaN.  A wave with such a V row
+    // works its rows again, each over its own keys; looked for only where the output
+    // is not finite (a NaN from a visible key costs the look, not the rows).  Above
+    // head_dim 128 only, where the per-pair kernel never read such a key: it is
+    // free there (16 / 8 heads d256 N = 1021 39.5 us either way), at 128 it takes 0.7%
+    // of 472 us, and the kernels beside it do as this one
+    if constexpr (D > 128) {
+        float z4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int d = 0; d < DB; d++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) z4[i & 3] = fmaf(0.f, o[d][i], z4[i & 3]);
+        float z = (z4[0] + z4[1]) + (z4[2] + z4[3]);
+        bool hidden = false;
+        if (__builtin_expect(__any(z != 0.f), 0)) {
+            z = 0.f;
+#pragma unroll 1
+            for (int t = max(mask_from, k_beg), t_end = min(k_beg + nw * TK, kend); t < t_end; t++)
+#pragma unroll 1
+                for (int c = lane; c < hd; c += 64) z = fmaf(0.f, to_f32<DT>(vb[(int64_t)t * p.row_stride + c]), z);
+            hidden = __any(z != 0.f);
+        }
+        if (__builtin_expect(hidden, 0)) {
+#pragma unroll 1
+            for (int r = r0; r < min(r0 + 32, R); r++) {
+                const int t = r / G;
+                const int64_t at = (int64_t)t * p.H + kvh * G + (r - t * G);
+                float oc[D / 64], m, l;
+                row_by_hand<D, DT>(p, p.q + at * hd, kb, vb, hd, k_beg, min(lim(t), kend), oc, m, l);
+                const float inv = l > 0.f ? 1.f / l : 0.f;
+                const int64_t slot_at = SPLIT ? at * p.ksplit + ks_id : at;
+                if (SPLIT && lane == 0) *reinterpret_cast<f32x2v_t*>(p.ws_ml + slot_at * 2) = f32x2v_t{m, l};
+                void* base = SPLIT ? static_cast<void*>(p.ws_o) : p.out;
+#pragma unroll
+                for (int c = 0; c < D / 64; c++)
+                    if (lane + 64 * c < hd) store_out<SDT>(base, slot_at * hd + lane + 64 * c, oc[c] * inv);
+            }
+            return;
+        }
+    }
+
     // ---- store.  Lane: row c32, columns 32d + 8a + 4h + i in o[d][4a + i]
     if (r0 + c32 >= R) return;
     const float l = sum_x32(l_part);
@@ -506,9 +598,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1
     const int64_t orow = (int64_t)tok * p.H + kvh * G + hi;
     if (SPLIT && h == 0)
         *reinterpret_cast<f32x2v_t*>(p.ws_ml + (orow * p.ksplit + ks_id) * 2) = f32x2v_t{m_run, l};
-    // partials: fp16 up to head_dim 128 (a convex combination of V rows, inside
-    // V's +-65504), fp32 above
-    constexpr int SDT = SPLIT ? (D > 128 ? DT_F32 : DT_F16) : OUT_DT;
     char* dst = SPLIT ? reinterpret_cast<char*>(p.ws_o) + (orow * p.ksplit + ks_id) * hd * (SDT == DT_F32 ? 4 : 2)
                       : static_cast<char*>(p.out) + orow * hd * (SDT == DT_F32 ? 4 : 2);
 #pragma unroll

@@ -111,6 +111,30 @@ def test_rows_climbing_scores(device, N, H, Hk, D, dtype):
     check(c, device, f"climbing scores, head_dim {D}")
 
 
+# a later token's V that is not finite: the rows before it, whose weight for it is
+# 0, do not take it in.  Token positions in the first and last tile of a wave, one
+# past a tile, the last one (whose row fills up the tile), after a context and with
+# split key ranges
+@pytest.mark.parametrize("N,H,Hk,D,start,at", [
+    (150, 16, 8, 256, 0, 5), (150, 16, 8, 256, 0, 149), (300, 8, 8, 256, 0, 33), (130, 32, 2, 256, 33, 65),
+    (257, 6, 2, 200, 63, 95), (140, 4, 1, 256, 1000, 77), (33, 14, 2, 248, 900, 32), (5, 16, 8, 256, 1501, 2),
+])
+@pytest.mark.parametrize("dtype", [C.F16, C.BF16])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_wide_rows_hidden_v(device, N, H, Hk, D, start, at, dtype, bad):
+    c = C.prefill_case(1900 + N + D, N, H, Hk, D, start, dtype)
+    C.say(f"prefill rows, V not finite N={N} H={H} Hk={Hk} D={D} start={start} at={at} dtype={dtype} {bad}")
+    q, k, v = (C.to_dev(c[x], dtype, device) for x in ("qb", "kb", "vb"))
+    kvh, G = Hk - 1, H // Hk
+    v[start + at, kvh] = bad
+    out = mugen_amd.flash_prefill_attention(q, k, v, start, out_dtype=torch.float32).cpu().numpy()
+    ref = C.prefill_ref(c, nthreads=16)  # of the finite V
+    C.assert_close(out[:at], ref[:at], "rows before the token")
+    if kvh:
+        C.assert_close(out[:, :kvh * G], ref[:, :kvh * G], "the other kv heads")
+    assert not np.isfinite(out[at:, kvh * G:]).any(), "rows that see it"
+
+
 def exact(q, k, v):
     """Causal attention over a prompt in 64 bits, head by head."""
     N, H, D = q.shape
