@@ -9,7 +9,6 @@ import numpy as np
 import pytest
 import torch
 
-import mugen_amd
 from mugen_amd import _capi
 from mugen_amd import attention as A
 from tests import cases as C
@@ -36,12 +35,26 @@ def planned(ws, size, per, bound):
     return None if chunk == -1 else chunk
 
 
-@pytest.mark.parametrize("B,H,Hk,D,hi,cache", [
-    (1, 8, 8, 64, 700, 8192), (1, 7, 1, 128, 1, 6000), (1, 16, 16, 64, 6000, 6000), (4, 32, 32, 64, 777, 2048), (8, 16, 16, 64, 900, 1024), (5, 28, 4, 128, 1500, 4096),
-    (16, 16, 4, 128, 300, 1024), (64, 4, 4, 64, 400, 512), (65, 3, 1, 64, 500, 640), (127, 2, 2, 64, 130, 256),
-    (3, 8, 2, 256, 900, 2048), (2, 4, 2, 96, 64, 65),
+def check_planned(chunk, on_device=True):
+    if on_device:
+        assert chunk is not None and chunk > 0 and chunk % 32 == 0, f"the device plan is taken: {chunk}"
+    else:
+        assert chunk is None, f"the static plan stays: {chunk}"
+
+
+# one guess up to 4 and up to 8 sequences, a search above, past the wave's 64
+# lanes, head_dim 256 (half the round), padded heads; then caches whose static plan
+# has chunks of 128 tokens or less, which stays
+@pytest.mark.parametrize("B,H,Hk,D,hi,cache,on_device", [
+    (1, 8, 8, 64, 700, 8192, True), (1, 7, 1, 128, 1, 6000, True), (1, 16, 16, 64, 6000, 6000, True),
+    (4, 32, 32, 64, 777, 2048, True), (8, 16, 16, 64, 900, 1024, True), (5, 28, 4, 128, 1500, 4096, True),
+    (16, 16, 4, 128, 300, 2048, True), (64, 4, 4, 64, 400, 512, True), (65, 3, 1, 64, 500, 2048, True),
+    (127, 2, 2, 64, 130, 1024, True), (3, 8, 2, 256, 900, 8192, True), (16, 8, 8, 256, 400, 512, True),
+    (2, 4, 2, 96, 64, 8192, True), (7, 8, 4, 40, 1000, 4096, True),
+    (16, 16, 4, 128, 300, 1024, False), (65, 3, 1, 64, 500, 640, False), (127, 2, 2, 64, 130, 256, False),
+    (3, 8, 2, 256, 900, 2048, False), (2, 4, 2, 96, 64, 65, False),
 ])
-def test_gqa_plan_on_device(device, B, H, Hk, D, hi, cache):
+def test_gqa_plan_on_device(device, B, H, Hk, D, hi, cache, on_device):
     lens = lens_of(B, hi, B + hi)
     c = C.gqa_decode_case(2100 + B, B, H, Hk, D, lens, max_T=cache, dtype=C.F16)
     ref = C.gqa_decode_ref(c, nthreads=16)
@@ -49,22 +62,33 @@ def test_gqa_plan_on_device(device, B, H, Hk, D, hi, cache):
     sl = torch.from_numpy(lens).to(device)
     C.say(f"gqa_decode without host lengths B={B} Hk={Hk} D={D} lens<={hi} cache={cache}")
     out = Guarded((B, H, D), torch.float32, device)
+    L = _capi.lib()
     a = A.gqa_decode_args(q, k, v, sl, out.t, cache)
-    need = _capi.lib().mugen_attn_gqa_decode_workspace_size(ctypes.byref(a))
+    need = L.mugen_attn_gqa_decode_workspace_size(ctypes.byref(a))
     host = np.full(B, cache, np.int32)  # every sequence full: the plan for max_seq_len
     a.seq_lens_host = host.ctypes.data
-    static = _capi.lib().mugen_attn_gqa_decode_workspace_size(ctypes.byref(a))
+    static = L.mugen_attn_gqa_decode_workspace_size(ctypes.byref(a))
+    a.seq_lens_host = None
+    padded = 64 if D <= 64 else 128 if D <= 128 else 256
     for size in (need, static):
         ws = guarded_ws(size, device)
+        ws.t.fill_(255)
         out.t.zero_()
-        mugen_amd.attention_decode(q, k, v, sl, cache, out=out.t, workspace=ws.t if size else None)
+        _capi.check(L.mugen_attn_gqa_decode(ctypes.byref(a), ctypes.c_void_p(ws.t.data_ptr()) if size else None, size,
+                                            A._stream(device)))
         assert out.intact() and ws.intact(), "guard band overwritten"
         C.assert_close(out.t.cpu().numpy(), ref, f"gqa plan on device, workspace {size}")
+        if size == need:
+            check_planned(planned(ws, need, B * H * (padded * 4 + 8), min(32, -(-cache // 64))), on_device)
 
 
-@pytest.mark.parametrize("B,H,q_len,hi,cache", [(1, 16, 1, 1000, 8192), (8, 128, 1, 700, 2048), (3, 128, 5, 600, 1024),
-                                                (64, 16, 1, 90, 128), (65, 16, 1, 70, 96), (2, 16, 16, 333, 4096)])
-def test_mla_plan_on_device(device, B, H, q_len, hi, cache):
+@pytest.mark.parametrize("B,H,q_len,hi,cache,on_device", [
+    (1, 16, 1, 1000, 8192, True), (4, 128, 1, 3000, 8192, True), (8, 128, 1, 700, 8192, True),
+    (5, 128, 1, 6000, 6000, True), (3, 128, 5, 600, 4096, True), (7, 16, 3, 500, 8192, True),
+    (64, 16, 1, 90, 1024, True), (65, 16, 1, 70, 1024, True), (33, 128, 1, 200, 1024, True), (2, 16, 16, 333, 8192, True),
+    (8, 128, 1, 700, 2048, False), (3, 128, 5, 600, 1024, False), (64, 16, 1, 90, 128, False),
+    (65, 16, 1, 70, 96, False), (2, 16, 16, 333, 4096, False)])
+def test_mla_plan_on_device(device, B, H, q_len, hi, cache, on_device):
     lens = np.maximum(lens_of(B, hi, B + hi), 0 if q_len == 1 else q_len).astype(np.int32)
     c = C.mla_case(2200 + B, B, q_len, H, lens, max_T=cache, q_dtype=C.F32, lat_dtype=C.F16)
     ref = C.mla_ref(c, nthreads=16)
@@ -72,17 +96,23 @@ def test_mla_plan_on_device(device, B, H, q_len, hi, cache):
     sl = torch.from_numpy(lens).to(device)
     C.say(f"mla_decode without host lengths B={B} H={H} q_len={q_len} lens<={hi} cache={cache}")
     out = Guarded((B, q_len, H, 512), torch.float32, device)
+    L = _capi.lib()
     a = A.mla_args(q, lat, sl, out.t, cache, C.MLA_SCALE)
-    need = _capi.lib().mugen_attn_mla_decode_workspace_size(ctypes.byref(a))
+    need = L.mugen_attn_mla_decode_workspace_size(ctypes.byref(a))
     host = np.full(B, cache, np.int32)
     a.seq_lens_host = host.ctypes.data
-    static = _capi.lib().mugen_attn_mla_decode_workspace_size(ctypes.byref(a))
+    static = L.mugen_attn_mla_decode_workspace_size(ctypes.byref(a))
+    a.seq_lens_host = None
+    R = q_len * H
     for size in (need, static):
         ws = guarded_ws(size, device)
+        ws.t.fill_(255)
         out.t.zero_()
-        mugen_amd.mla_attention(q, lat, sl, cache, scale=C.MLA_SCALE, out=out.t, workspace=ws.t)
+        _capi.check(L.mugen_attn_mla_decode(ctypes.byref(a), ctypes.c_void_p(ws.t.data_ptr()), size, A._stream(device)))
         assert out.intact() and ws.intact(), "guard band overwritten"
         C.assert_close(out.t.cpu().numpy(), ref, f"mla plan on device, workspace {size}")
+        if size == need:
+            check_planned(planned(ws, need, B * ((R + 15) // 16 * 16 * 1024 + R * 8), min(32, -(-cache // 32))), on_device)
 
 
 # the store rounds a sequence's Q4 and f16 tokens up to splits on their own: batches
@@ -124,8 +154,7 @@ def test_q4_plan_on_device(device, H, Hk, D, lens, keep, cache):
     C.say(f"gqa_decode_q4 without host lengths B={B} Hk={Hk} D={D} lens<={T} cache={cache}")
     _capi.check(L.mugen_attn_gqa_decode_q4(ctypes.byref(a), ctypes.c_void_p(ws.t.data_ptr()), need, A._stream(device)))
     assert out.intact() and ws.intact(), "guard band overwritten"
-    chunk = planned(ws, need, B * H * (D * 4 + 8), min(32, -(-cache // 64)) + 1)
-    assert chunk is not None and chunk > 0 and chunk % 32 == 0, "the device plan is taken"
+    check_planned(planned(ws, need, B * H * (D * 4 + 8), min(32, -(-cache // 64)) + 1))
     C.assert_close(out.t.cpu().numpy(), oracle_decode(q, k, v, lens, nq, H, Hk, D), f"q4 plan on device B={B}")
 
 
