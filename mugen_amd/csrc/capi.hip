@@ -194,9 +194,17 @@ static int gqa_budget(const mugen_attn_gqa_decode_args* a) { return a->head_dim 
 // 256 260); 40 sequences 210 -> 177, 24 at 16 / 8 heads d256 240 -> 185, 64 at d64
 // 157 -> 129.  From 1.35 times the mean: equal lengths (363 us unsplit, 396 in
 // 1024s) and 48 sequences at 28 / 4 heads (1.23 times: 94.6 against 98.6) stay
-// in one round.  Needs the host lengths.
-constexpr int kGqaDeepChunk = 1024;
-static bool gqa_deep(const mugen_attn_gqa_decode_args* a, int chunk, int64_t budget) {
+// in one round.  Needs the host lengths.  Past one round unsplit (65 sequences at 8
+// kv heads) each stays one item.
+// The 4-bit store, whose second kind of split takes a large part of the round
+// (chunk against the mean 1.3 with equal lengths already): 64 sequences of
+// 512..8191 at 28 / 4 heads 161 -> 77 us, 24 at 32 / 8 80 -> 60, 32 equal ones 184 ->
+// 117.  Chunks up to 1792 gain only where they are past twice the mean: 12 of
+// 3000..8191 at 32 / 8 heads, chunk 1344, 39 -> 43, 24 at 28 / 4 37 -> 39, 128 at 4 / 1,
+// chunk 1792, 45 -> 46; 100 of 100..3000 at 8 / 2, chunk 1568, 2.4 times, 41 -> 34, 32
+// of 512..8191 at 28 / 4, chunk 1920, 48.6 -> 47.9
+constexpr int kGqaDeepChunk = 1024, kGqaDeepStoreChunk = 1792;
+static bool gqa_deep(const mugen_attn_gqa_decode_args* a, int chunk, int64_t budget, bool store) {
     if (!a->seq_lens_host || chunk <= kGqaDeepChunk) return false;
     int64_t sum = 0;
     int longest = 0;
@@ -205,7 +213,8 @@ static bool gqa_deep(const mugen_attn_gqa_decode_args* a, int chunk, int64_t bud
         sum += T;
         longest = std::max(longest, T);
     }
-    return (double)std::min(chunk, longest) * (double)budget > 1.35 * (double)sum * a->n_kv_heads;
+    const double least = store && chunk <= kGqaDeepStoreChunk ? 2.0 : 1.35;
+    return (double)std::min(chunk, longest) * (double)budget > least * (double)sum * a->n_kv_heads;
 }
 
 // deep: false keeps the one-round plan (whose partials may fit a workspace
@@ -236,7 +245,7 @@ static int gqa_chunk(const mugen_attn_gqa_decode_args* a, int extra = 0, bool de
         else lo = mid + q;
     }
     if (gqa_items(a, lo, extra) > budget) lo = hi;
-    return deep && gqa_deep(a, lo, budget) ? std::max(kGqaDeepChunk, cmin) : lo;
+    return deep && gqa_deep(a, lo, budget, extra > 0) ? std::max(kGqaDeepChunk, cmin) : lo;
 }
 
 static int gqa_validate(const mugen_attn_gqa_decode_args* a, bool ring_store = false) {
