@@ -379,7 +379,7 @@ private:
         d.scale = s_.scale;
         d.kv_dtype = s_.kv_dtype;
         d.out_dtype = s_.out_dtype;
-        d.seq_lens_host = nullptr;  // the grid is planned for max_seq_len: one plan serves every step
+        d.seq_lens_host = nullptr;  // planned on the device from its lengths: one call serves every step
         return d;
     }
 
@@ -655,7 +655,7 @@ private:
         d.max_seq_len = s_.max_seq_len;
         d.scale = s_.scale;
         d.out_dtype = s_.out_dtype;
-        d.seq_lens_host = nullptr;  // planned for max_seq_len: one plan serves every step
+        d.seq_lens_host = nullptr;  // planned on the device from its lengths: one call serves every step
         return d;
     }
 

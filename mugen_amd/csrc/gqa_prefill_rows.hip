@@ -42,11 +42,13 @@
 // ring slots (the loop unrolled over the ring) 1% faster at N = 8192 for four
 // times the code.
 //
-// Bound at head_dim 256: MFMA issue of one wave per SIMD (64 MFMAs of 32
-// cycles per 64 keys and 32 rows), ~1.3 us per pair of tiles measured against
-// 0.9 of MFMAs.  16 / 8 heads, f16, one prompt: N = 1021 523 -> 38 us (16 ->
-// 226 TFLOP/s), N = 2048 1890 -> 70 us, 100 tokens after 1500 172 -> 26 us;
-// before, every (token, kv head) pair walked its keys in its own workgroup.
+// Bound at head_dim 256: the chain of one wave per SIMD, on half of them (16 / 8
+// heads N = 1021: 128 workgroups, the longest 32 tiles at ~1.1 us, of which the
+// matrix pipes take 0.45 (32 MFMAs of 32 cycles); a wave issues in half of its
+// cycles, waits on memory or LDS for 28% and for its turn for 23%).  16 / 8 heads,
+// f16, one prompt: N = 1021 523 -> 38 us (16 -> 226 TFLOP/s), N = 2048 1890 -> 70 us,
+// 100 tokens after 1500 172 -> 26 us; before, every (token, kv head) pair walked its
+// keys in its own workgroup.
 #include "common.h"
 #include "kernels.h"
 
