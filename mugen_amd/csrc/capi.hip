@@ -735,13 +735,6 @@ static bool gqa_prefill_v16_capable(const mugen_attn_gqa_prefill_args* a) {
     return a->head_dim <= 128 && a->dtype == DT_BF16;
 }
 
-// head_dim above 128, keys not split: up to this many (token, kv head) pairs
-// (one round of workgroups) run one to a workgroup, whose four waves share
-// the pair's keys; past it the flattened-row kernel.  16 / 8 heads, us,
-// per pair / flattened: N = 32 5.4 / 7.1, 64 9.9 / 8.5, 256 53 / 14.8; 16 / 4
-// heads at head_dim 192, N = 64 6.4 / 11.3, 512 86 / 26
-constexpr int kPrefillWideItems = 256;
-
 // The automatic choice of the short-prompt kernel: the whole kv range fits
 // on chip, from 384 visible keys on (below that the per-block kernel's
 // shorter load phase wins: Llama-3.2-1B N = 128 4.4 against 4.9 us; N = 256
@@ -884,7 +877,8 @@ int mugen_attn_gqa_prefill(const mugen_attn_gqa_prefill_args* a, void* stream) {
             p.ws_ml = align256(a->workspace);
             p.ws_o = reinterpret_cast<uint16_t*>(p.ws_ml + prefill_partials_at((size_t)a->n_tokens * a->n_heads * split.ksplit));
         }
-        if (p.ksplit > 1 || (int64_t)a->n_tokens * a->n_kv_heads > kPrefillWideItems) {
+        if (p.ksplit > 1 ||
+            prefill_wide_rows_default(a->n_tokens, a->start_pos, a->causal, p.G, a->n_kv_heads, a->head_dim)) {
             hipError_t e = launch_gqa_prefill_rows(p, a->n_kv_heads, a->dtype, a->out_dtype, st, active_timer());
             if (e == hipSuccess && p.ksplit > 1) e = launch_gqa_prefill_combine(p, a->out_dtype, st, active_timer());
             return hip_status(e, "gqa_prefill launch");
@@ -911,8 +905,6 @@ int mugen_attn_gqa_prefill(const mugen_attn_gqa_prefill_args* a, void* stream) {
         d.max_T = a->kv_len;
         d.pf_start = a->start_pos;
         d.pf_causal = a->causal ? 1 : 0;
-        if ((int64_t)a->n_tokens * a->n_kv_heads > INT32_MAX)
-            return fail(MUGEN_ATTN_E_UNSUPPORTED, "gqa_prefill: n_tokens * n_kv_heads too large");
         return hip_status(launch_gqa_prefill_wide(d, a->dtype, a->out_dtype, st, active_timer()),
                           "gqa_prefill launch");
     }

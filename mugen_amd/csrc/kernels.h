@@ -77,8 +77,8 @@ struct GqaDecodeParams {
 hipError_t launch_gqa_decode(const GqaDecodeParams& p, int nwg, int D, int kv_dt, int out_dt, hipStream_t st,
                              KernelTimer* t);
 hipError_t launch_gqa_decode_q4(const GqaDecodeParams& p, int nwg, int D, int out_dt, hipStream_t st, KernelTimer* t);
-// a short prompt at head_dim 129..256 (up to kPrefillWideItems (token, kv
-// head) pairs, no key split) through the decode kernel's prompt mode
+// a short prompt at head_dim 129..256 (few (token, kv head) pairs, no key split:
+// prefill_wide_rows_default) through the decode kernel's prompt mode
 // (p.B = query tokens, one split, p.pf_start / p.pf_causal set)
 hipError_t launch_gqa_prefill_wide(const GqaDecodeParams& p, int kv_dt, int out_dt, hipStream_t st, KernelTimer* t);
 

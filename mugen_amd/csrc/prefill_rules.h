@@ -1,5 +1,4 @@
-// prefill_rules.h -- which prefill kernel takes a prompt at head_dim up to 128,
-// and where a split call's partials lie.  Plain integer C++, so that
+// prefill_rules.h -- which prefill kernel takes a prompt, and where a split call's partials lie.  Plain integer C++, so that
 // tests/cpp/prefill_rules_check.cpp prints the same on the host.
 #pragma once
 #include <cstddef>
@@ -57,6 +56,21 @@ inline bool prefill_rows_default(int n_tokens, int start_pos, bool causal, int G
         least = 800;
     }
     return wgs >= least;
+}
+
+// head_dim above 128, keys not split: up to one round of (token, kv head) pairs,
+// at head_dim below 256 two, run one pair to a workgroup, whose four waves share
+// the pair's keys; past it the flattened-row kernel, which pads every head to 256
+// columns where a pair moves head_dim.  us, per pair / flattened: 16 / 8 heads d256
+// N = 32 5.4 / 7.1, 64 9.9 / 8.5, 256 53 / 14.8; d256 260 to 512 pairs 0.75 to 1.0 of
+// the pairs' time at 1 to 16 kv heads.  d136: 1 / 1 heads N = 290 15.9 / 19.7, 600
+// 32 / 28; 4 / 4 110 10.5 / 13.0, 150 19 / 15; d192: 4 / 4 110 11.1 / 13.5, 150 20 / 16.
+// With 64 heads and more the blocks fill sooner: 128 / 16 heads d136 N = 17 11.8 /
+// 10.5, 64 / 8 33 11.8 / 11.2, 64 / 16 17 10.7 / 10.1 (after as many tokens 11.1 / 11.4)
+inline bool prefill_wide_rows_default(int n_tokens, int start_pos, bool causal, int G, int n_kv_heads, int head_dim) {
+    const bool level = !causal || start_pos >= n_tokens;
+    const bool early = head_dim == 256 || (G * n_kv_heads >= 64 && (G >= 8 || !level));
+    return (int64_t)n_tokens * n_kv_heads > (early ? 256 : 512);
 }
 
 // Key splits: floats from the (max, sum) pairs, at a 256-byte boundary of the

@@ -18,7 +18,10 @@ int main(int argc, char**) {
     }
     int n, start, causal, h, hk, d;
     while (std::scanf("%d %d %d %d %d %d", &n, &start, &causal, &h, &hk, &d) == 6)
-        std::puts(prefill_rows_default(n, start, causal != 0, h / hk, hk, d) ? "rows"
+        if (d > 128)
+            std::puts(prefill_wide_rows_default(n, start, causal != 0, h / hk, hk, d) ? "rows" : "pairs");
+        else
+            std::puts(prefill_rows_default(n, start, causal != 0, h / hk, hk, d) ? "rows"
                   : prefill_ws_default(n, h / hk, d)                         ? "ws"
                                                                              : "block");
     return 0;

@@ -39,6 +39,12 @@ def choose(tmp_path_factory):
     (10300, 8, 1, 64, "ws"), (12800, 8, 1, 64, "rows"),
     # 8 heads per kv head, full slots
     (5180, 16, 2, 128, "ws"), (6144, 16, 2, 128, "rows"), (2620, 32, 4, 128, "rows"),
+    # above head_dim 128: a workgroup per (token, kv head) pair, one round of them at
+    # 256, two at the padded widths, one with many heads
+    (32, 16, 8, 256, "pairs"), (33, 16, 8, 256, "rows"), (1021, 16, 8, 256, "rows"), (256, 1, 1, 256, "pairs"),
+    (257, 1, 1, 256, "rows"), (300, 1, 1, 136, "pairs"), (513, 1, 1, 136, "rows"), (64, 16, 8, 192, "pairs"),
+    (65, 16, 8, 192, "rows"), (128, 16, 4, 192, "pairs"), (129, 16, 4, 192, "rows"), (17, 128, 16, 136, "rows"),
+    (33, 64, 8, 192, "rows"), (17, 64, 16, 192, "rows"),
 ])
 def test_prompt_kernel(choose, N, H, Hk, D, kernel):
     assert choose(N, 0, 1, H, Hk, D) == kernel
@@ -48,6 +54,7 @@ def test_prompt_kernel(choose, N, H, Hk, D, kernel):
 @pytest.mark.parametrize("N,H,Hk,D,kernel", [
     (2933, 28, 4, 128, "ws"), (3518, 28, 4, 128, "rows"), (2568, 32, 4, 128, "ws"), (3072, 32, 4, 128, "ws"), (4400, 32, 4, 128, "rows"),
     (2048, 16, 8, 64, "rows"), (16384, 2, 1, 64, "block"), (20500, 4, 1, 64, "rows"), (3421, 24, 4, 128, "rows"), (2926, 28, 4, 64, "rows"),
+    (17, 64, 16, 192, "pairs"), (33, 64, 8, 192, "rows"), (33, 16, 8, 256, "rows"),
 ])
 def test_level_chunk_kernel(choose, N, H, Hk, D, kernel):
     assert choose(N, N, 1, H, Hk, D) == kernel and choose(N, 0, 0, H, Hk, D) == kernel
