@@ -317,14 +317,26 @@ static int stride_bound(int max_seq_len, int qmin, int extra) {
 // work).  The longest sequence gets as many splits as the workspace has room
 // for, up to stride_bound, which the workspace sizes cover; below the static
 // plan's own count, and in large batches, whose sequences fill half a round
-// unsplit, the static plan stays; also where its chunk is 128 tokens or less
-// (one sequence of 700 tokens in a 4096-token cache: 6.0 us static, 6.2 planned,
-// of 3000 in 8192, chunk 256: 8.9 and 7.5).
+// unsplit, the static plan stays.
 static bool gqa_device_plan(const mugen_attn_gqa_decode_args* a, int extra) {
     return !a->seq_lens_host && a->num_splits <= 0 && (int64_t)a->batch * a->n_kv_heads * 2 <= gqa_budget(a) &&
            stride_bound(a->max_seq_len, kGqaChunkMin, extra) > 1;
 }
-constexpr int kPlanStaticChunk = 128;
+// Planning takes the two kernels 0.3 to 1.4 us, so not where the static plan's chunk
+// leaves little to gain: of 128 tokens or less, and of up to 256 for up to 4
+// sequences, head_dim up to 128, whose splits come near the round (us, static /
+// planned in full caches, at 5..40%: 32 / 8 heads d64, 4 sequences in 4096-token
+// caches 9.4 / 10.8, 7.4 / 8.2; d128 16.2 / 17.8, 9.6 / 10.0; one 28 / 4 d128 in 8192 stays
+// planned, 9.2 / 9.6, 8.9 / 7.4).  The store, which plans for two runs of a sequence,
+// also where a few pairs leave the round empty (14 / 2 d64, one in 8192 8.1 / 9.3, 8 /
+// 7.9; 28 / 4 d128, 4 in 4096 11.6 / 12.9, 11.4 / 11.9)
+constexpr int kPlanStaticChunk = 128, kPlanStaticFew = 256;
+static bool gqa_plan_pays(const mugen_attn_gqa_decode_args* a, int chunk, bool store) {
+    if (chunk <= kPlanStaticChunk) return false;
+    if (a->batch > 4 || a->head_dim > 128 || chunk > kPlanStaticFew) return true;
+    const int pairs = a->batch * a->n_kv_heads;
+    return store ? pairs > 6 && pairs < 16 : pairs <= 16;
+}
 constexpr size_t kPlanBytes = 256;  // the planned chunk, after the partials
 // most splits per sequence whose partials (one split's: `per` bytes) fit a
 // workspace beside the alignment and the plan
@@ -590,7 +602,7 @@ int mugen_attn_gqa_decode_q4(const mugen_attn_gqa_decode_q4_args* a, void* ws, s
     size_t need = gqa_q4_ws(a, chunk, &splits);
     if (ws_bytes < need) need = gqa_q4_ws(a, chunk = gqa_chunk(&g, 1, false), &splits);
     const int fit = ws ? plan_fit(ws_bytes, gqa_split_bytes(&g), stride_bound(a->max_seq_len, kGqaChunkMin, 1)) : 0;
-    const bool dev = gqa_device_plan(&g, 1) && chunk > kPlanStaticChunk && fit >= splits;
+    const bool dev = gqa_device_plan(&g, 1) && gqa_plan_pays(&g, chunk, true) && fit >= splits;
     if (dev) need = gqa_q4_ws(a, chunk, &splits, fit);
     if (!ws || ws_bytes < need)
         return fail(MUGEN_ATTN_E_WORKSPACE, "gqa_decode_q4: workspace of %zu bytes required, %zu given", need,
@@ -653,7 +665,7 @@ int mugen_attn_gqa_decode(const mugen_attn_gqa_decode_args* a, void* ws, size_t 
     size_t need = gqa_ws(a, chunk, &splits);
     if (!ws || ws_bytes < need) need = gqa_ws(a, chunk = gqa_chunk(a, 0, false), &splits);
     const int fit = ws ? plan_fit(ws_bytes, gqa_split_bytes(a), stride_bound(a->max_seq_len, kGqaChunkMin, 0)) : 0;
-    const bool dev = gqa_device_plan(a, 0) && chunk > kPlanStaticChunk && fit > 1 && fit >= splits;
+    const bool dev = gqa_device_plan(a, 0) && gqa_plan_pays(a, chunk, false) && fit > 1 && fit >= splits;
     if (dev) need = gqa_ws(a, chunk, &splits, fit);
     if (need > 0 && (!ws || ws_bytes < need))
         return fail(MUGEN_ATTN_E_WORKSPACE, "gqa_decode: workspace of %zu bytes required, %zu given", need,

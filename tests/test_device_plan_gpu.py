@@ -44,7 +44,7 @@ def check_planned(chunk, on_device=True):
 
 # one guess up to 4 and up to 8 sequences, a search above, past the wave's 64
 # lanes, head_dim 256 (half the round), padded heads; then caches whose static plan
-# has chunks of 128 tokens or less, which stays
+# has chunks of 128 tokens or less, or of 256 for a few sequences, which stays
 @pytest.mark.parametrize("B,H,Hk,D,hi,cache,on_device", [
     (1, 8, 8, 64, 700, 8192, True), (1, 7, 1, 128, 1, 6000, True), (1, 16, 16, 64, 6000, 6000, True),
     (4, 32, 32, 64, 777, 2048, True), (8, 16, 16, 64, 900, 1024, True), (5, 28, 4, 128, 1500, 4096, True),
@@ -52,7 +52,7 @@ def check_planned(chunk, on_device=True):
     (127, 2, 2, 64, 130, 1024, True), (3, 8, 2, 256, 900, 8192, True), (16, 8, 8, 256, 400, 512, True),
     (2, 4, 2, 96, 64, 8192, True), (7, 8, 4, 40, 1000, 4096, True),
     (16, 16, 4, 128, 300, 1024, False), (65, 3, 1, 64, 500, 640, False), (127, 2, 2, 64, 130, 256, False),
-    (3, 8, 2, 256, 900, 2048, False), (2, 4, 2, 96, 64, 65, False),
+    (3, 8, 2, 256, 900, 2048, False), (2, 4, 2, 96, 64, 65, False), (4, 8, 8, 64, 900, 4096, False),
 ])
 def test_gqa_plan_on_device(device, B, H, Hk, D, hi, cache, on_device):
     lens = lens_of(B, hi, B + hi)
@@ -121,9 +121,9 @@ def test_mla_plan_on_device(device, B, H, q_len, hi, cache, on_device):
 # shows a work item that nobody took
 @pytest.mark.parametrize("H,Hk,D,lens,keep,cache", [
     (8, 8, 64, [4600, 5853, 3424, 4723, 5733, 5020, 4463, 3623], 256, 8192),
-    (8, 4, 64, [3054] * 4, 256, 4096),
+    (16, 8, 64, [6100] * 4, 256, 8192),
     (8, 8, 64, [5000] * 6, 256, 8192),
-    (8, 8, 64, [7168] * 2, 256, 8192),
+    (16, 16, 64, [7168] * 2, 256, 8192),
     (16, 8, 128, [2900], 100, 8192),
     (2, 2, 256, [8000, 1, 0, 1024, 1024, 1024, 1024], 256, 8192),
     (16, 16, 64, [1000 + 37 * i for i in range(16)], 200, 2048),
