@@ -286,8 +286,8 @@ __device__ __forceinline__ int wave_scan_i32(int v) {
 // -- mult items per split, count(j, c) splits of sequence j at chunk c -- fits
 // `budget` workgroups (the host sees to KINDS B mult <= budget); every wave
 // computes the same one.  units(j): 32-token units of sequence j.  The kernels
-// wait for it, so up to 8 sequences take one guess (plan_few), and more the
-// smallest chunk to 1/16, searched from that guess.
+// wait for it, so up to 8 sequences take one guess (plan_few), and more a
+// search from it (plan_many).
 template <int KINDS, typename Units, typename Count>
 __device__ __forceinline__ int plan_chunk_device(int B, int mult, int budget, int cmin, int cap,
                                                  Units units, Count count) {
@@ -318,9 +318,9 @@ __device__ __forceinline__ int plan_chunk_device(int B, int mult, int budget, in
         };
         auto add = [](int a, int b) { return a + b; };
         const int l = lane & 7, u = l < B ? units(l) : 0;
-        const int mx = fold(u, [](int a, int b) { return max(a, b); });
+        const int mx = fold(u, [](int a, int b) { return max(a, b); }), sum = fold(u, add);
         return 32 * __builtin_amdgcn_readfirstlane(
-                        plan_few<KINDS>(B, mult, budget, plan_by_cap(mx, cmin, cap), cap, fold(u, add), mx,
+                        plan_few<KINDS>(B, mult, budget, plan_by_cap(mx, cmin, cap), cap, sum, mx,
                                         [&](int x, float rx) { return fold(l < B ? count(l, x, rx) : 0, add); }));
     }
     int sum = 0, mx = 0;
@@ -331,13 +331,12 @@ __device__ __forceinline__ int plan_chunk_device(int B, int mult, int budget, in
     }
     sum = __builtin_amdgcn_readfirstlane(wave_sum_i32(sum));
     mx = -__builtin_amdgcn_readfirstlane(wave_min_i32(-mx));
-    const int c0 = __builtin_amdgcn_readfirstlane(
-        max(plan_by_cap(mx, cmin, cap), plan_div_up(sum * mult, budget - B * mult / 2) - 1));
-    return 32 * plan_grow(c0, mx, mult, budget, [&](int c, float rc) {
+    const int c0 = __builtin_amdgcn_readfirstlane(plan_by_cap(mx, cmin, cap));
+    return 32 * __builtin_amdgcn_readfirstlane(plan_many<KINDS>(B, mult, budget, c0, sum, mx, [&](int c, float rc) {
                int n = 0;
                for (int j = lane; j < B; j += 64) n += count(j, c, rc);
                return __builtin_amdgcn_readfirstlane(wave_sum_i32(n));
-           });
+           }));
 }
 
 // Work item -> sequence: sequence j has n(j) items, numbered in order; sets j

@@ -68,4 +68,23 @@ MUGEN_PLAN_FN int plan_few(int B, int mult, int budget, int c0, int cap, int sum
     return c;
 }
 
+// The plan of more sequences, a search: the longest sequence cut evenly at the
+// guess of half a split lost per sequence, where that fits (32 equal sequences
+// fill the round exactly with two halves each: 32 / 8 heads d128, full caches of
+// 8192, 222 -> 200 us against two thirds and one), else the smallest chunk to 1/16
+// from that guess.  A store whose two runs per sequence leave room for less than
+// half a split more each takes one split of each at once (32 / 8 heads, 32
+// sequences: the search took 4.7 of 42 us)
+template <int KINDS, typename Total>
+MUGEN_PLAN_FN int plan_many(int B, int mult, int budget, int c0, int sum, int mx, Total total) {
+    if (KINDS > 1 && (2 * KINDS + 1) * B * mult > 2 * budget) return plan_max(c0, mx);
+    const int c = plan_max(c0, plan_div_up(sum * mult, budget - KINDS * B * mult / 2) - 1);
+    const int ns = ceil_div_f(mx, c, plan_rcp(c));
+    if (mx > 0) {
+        const int even = plan_max(c0, ceil_div_f(mx, ns, plan_rcp(ns)));
+        if (total(even, plan_rcp(even)) * mult <= budget) return even;
+    }
+    return plan_grow(c, mx, mult, budget, total);
+}
+
 }  // namespace mugen_attn

@@ -32,6 +32,7 @@ struct Case {
     int kinds, mult, budget, cmin, cap;
     bool empty_counts;         // an empty sequence still has one split (GQA)
     std::vector<int> T, nq;    // tokens, of which quantised (kinds 2)
+    int longest = 1 << 30;     // the longest chunk that is good enough
 };
 
 int run_of(const Case& c, int j, int kind) {  // units of one run of a sequence
@@ -63,8 +64,8 @@ void check(const Case& c, const char* what) {
         chunk = c.kinds == 1 ? plan_few<1>(B, c.mult, c.budget, c0, c.cap, sum, mx, total)
                              : plan_few<2>(B, c.mult, c.budget, c0, c.cap, sum, mx, total);
     else
-        chunk = plan_grow(plan_max(c0, plan_div_up(sum * c.mult, c.budget - B * c.mult / 2) - 1), mx, c.mult, c.budget,
-                          total);
+        chunk = c.kinds == 1 ? plan_many<1>(B, c.mult, c.budget, c0, sum, mx, total)
+                             : plan_many<2>(B, c.mult, c.budget, c0, sum, mx, total);
     long items = 0;
     int most = 0;
     for (int j = 0; j < B; j++) {
@@ -76,7 +77,7 @@ void check(const Case& c, const char* what) {
     items *= c.mult;
     // workgroups of the launch: one round, or every slot of every sequence
     const long slots = c.cap + c.kinds - 1, wgs = std::min<long>(c.budget, (long)B * c.mult * slots);
-    if (chunk < c.cmin || items > wgs || most > slots) {
+    if (chunk < c.cmin || items > wgs || most > slots || chunk > c.longest) {
         violations++;
         if (violations <= 20) {
             std::printf("%s: kinds %d batch %d mult %d budget %d cap %d ulp %d: chunk %d, %ld items for %ld workgroups, "
@@ -107,6 +108,10 @@ int main(int argc, char** argv) {
         store({7168, 7168, 7168, 7168}, 4, 512, 32, 256, "4 equal sequences x 4 kv heads");
         store({8000, 1024, 1024, 1024, 1024, 1024, 1024, 1024}, 32, 512, 32, 256, "8 sequences x 32 kv heads");
         store(std::vector<int>(6, 5000), 8, 512, 32, 256, "6 equal sequences x 8 kv heads");
+        // equal sequences that fill the round exactly, cut in halves
+        check({1, 8, 512, 2, 32, true, std::vector<int>(32, 8192), {}, 128}, "32 full sequences x 8 kv heads");
+        check({1, 8, 256, 2, 32, true, std::vector<int>(16, 4096), {}, 64}, "16 full sequences x 8 kv heads");
+        check({1, 4, 512, 2, 32, true, std::vector<int>(32, 4096), {}, 32}, "32 full sequences x 4 kv heads");
         // every batch up to 64 that plans on the device, equal lengths and drawn
         // ones, every split cap that a workspace can leave
         const int budgets[] = {256, 512, 256};  // GQA above head_dim 128 and up to it, MLA

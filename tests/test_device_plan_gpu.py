@@ -50,7 +50,8 @@ def check_planned(chunk, on_device=True):
     (4, 32, 32, 64, 777, 2048, True), (8, 16, 16, 64, 900, 1024, True), (5, 28, 4, 128, 1500, 4096, True),
     (16, 16, 4, 128, 300, 2048, True), (64, 4, 4, 64, 400, 512, True), (65, 3, 1, 64, 500, 2048, True),
     (127, 2, 2, 64, 130, 1024, True), (3, 8, 2, 256, 900, 8192, True), (16, 8, 8, 256, 400, 512, True),
-    (2, 4, 2, 96, 64, 8192, True), (7, 8, 4, 40, 1000, 4096, True),
+    (2, 4, 2, 96, 64, 8192, True), (7, 8, 4, 40, 1000, 4096, True), (32, 8, 8, 64, 2048, 2048, True),
+    (16, 8, 8, 256, 1024, 1024, True),
     (16, 16, 4, 128, 300, 1024, False), (65, 3, 1, 64, 500, 640, False), (127, 2, 2, 64, 130, 256, False),
     (3, 8, 2, 256, 900, 2048, False), (2, 4, 2, 96, 64, 65, False), (4, 8, 8, 64, 900, 4096, False),
 ])
