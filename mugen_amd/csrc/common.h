@@ -281,15 +281,15 @@ __device__ __forceinline__ int wave_scan_i32(int v) {
 // The context-split plan from the lengths on the device, for calls without
 // host lengths (captured decode steps: one plan made for max_seq_len would
 // leave most workgroups without work in a cache that is not full).  A chunk of
-// 32-token units, at least cmin, that cuts the longest sequence into at most
+// 32-token units, at least cmin(units of the batch), that cuts the longest sequence into at most
 // `cap` splits (the store, KINDS 2: one more, see plan_few) and whose work list
 // -- mult items per split, count(j, c) splits of sequence j at chunk c -- fits
 // `budget` workgroups (the host sees to KINDS B mult <= budget); every wave
 // computes the same one.  units(j): 32-token units of sequence j.  The kernels
 // wait for it, so up to 8 sequences take one guess (plan_few), and more a
 // search from it (plan_many).
-template <int KINDS, typename Units, typename Count>
-__device__ __forceinline__ int plan_chunk_device(int B, int mult, int budget, int cmin, int cap,
+template <int KINDS, typename Least, typename Units, typename Count>
+__device__ __forceinline__ int plan_chunk_device(int B, int mult, int budget, Least cmin, int cap,
                                                  Units units, Count count) {
     const int lane = threadIdx.x & 63;
     if (B <= 4) {  // scalar loads, all at once (indices past B repeat the last sequence)
@@ -301,7 +301,7 @@ __device__ __forceinline__ int plan_chunk_device(int B, int mult, int budget, in
             sum += j < B ? u[j] : 0;
         }
         return 32 * __builtin_amdgcn_readfirstlane(plan_few<KINDS>(
-                        B, mult, budget, plan_by_cap(mx, cmin, cap), cap, sum, mx, [&](int x, float rx) {
+                        B, mult, budget, plan_by_cap(mx, cmin(sum), cap), cap, sum, mx, [&](int x, float rx) {
                             int n = 0;
 #pragma unroll
                             for (int j = 0; j < 4; j++)
@@ -320,7 +320,7 @@ __device__ __forceinline__ int plan_chunk_device(int B, int mult, int budget, in
         const int l = lane & 7, u = l < B ? units(l) : 0;
         const int mx = fold(u, [](int a, int b) { return max(a, b); }), sum = fold(u, add);
         return 32 * __builtin_amdgcn_readfirstlane(
-                        plan_few<KINDS>(B, mult, budget, plan_by_cap(mx, cmin, cap), cap, sum, mx,
+                        plan_few<KINDS>(B, mult, budget, plan_by_cap(mx, cmin(sum), cap), cap, sum, mx,
                                         [&](int x, float rx) { return fold(l < B ? count(l, x, rx) : 0, add); }));
     }
     int sum = 0, mx = 0;
@@ -331,7 +331,7 @@ __device__ __forceinline__ int plan_chunk_device(int B, int mult, int budget, in
     }
     sum = __builtin_amdgcn_readfirstlane(wave_sum_i32(sum));
     mx = -__builtin_amdgcn_readfirstlane(wave_min_i32(-mx));
-    const int c0 = __builtin_amdgcn_readfirstlane(plan_by_cap(mx, cmin, cap));
+    const int c0 = __builtin_amdgcn_readfirstlane(plan_by_cap(mx, cmin(sum), cap));
     return 32 * __builtin_amdgcn_readfirstlane(plan_many<KINDS>(B, mult, budget, c0, sum, mx, [&](int c, float rc) {
                int n = 0;
                for (int j = lane; j < B; j += 64) n += count(j, c, rc);

@@ -91,7 +91,7 @@ __device__ __forceinline__ int plan_gqa(const GqaDecodeParams& p) {
         return (T - min(clamp_len(p.n_q4[j], p.max_T), T) + 31) >> 5;
     };
     return plan_chunk_device<Q4 ? 2 : 1>(
-        p.B, p.Hk, p.budget, 2, Q4 ? p.num_splits - 1 : p.num_splits, [&](int j) { return Q4 ? q4u(j) + ring(j) : len(j); },
+        p.B, p.Hk, p.budget, [](int) { return 2; }, Q4 ? p.num_splits - 1 : p.num_splits, [&](int j) { return Q4 ? q4u(j) + ring(j) : len(j); },
         [&](int j, int c, float rc) {
             return max(1, Q4 ? ceil_div_f(q4u(j), c, rc) + ceil_div_f(ring(j), c, rc) : ceil_div_f(len(j), c, rc));
         });

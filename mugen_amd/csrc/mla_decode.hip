@@ -84,7 +84,7 @@ __device__ __forceinline__ int64_t blob_pair(const MlaParams& p, int b, int s, i
 // the device plan of this call (plan_chunk_device)
 __device__ __forceinline__ int plan_mla(const MlaParams& p) {
     auto len = [&](int j) { return (clamp_len(p.seq_lens[j], p.max_T) + 31) >> 5; };
-    return plan_chunk_device<1>(p.B, p.nrb, p.units, 1, p.num_splits, len,
+    return plan_chunk_device<1>(p.B, p.nrb, p.units, [&](int sum) { return plan_mla_least(sum, p.R); }, p.num_splits, len,
                              [&](int j, int c, float rc) { return ceil_div_f(len(j), c, rc); });
 }
 

@@ -13,6 +13,9 @@
 #ifndef MUGEN_PLAN_RCP
 #define MUGEN_PLAN_RCP(x) __builtin_amdgcn_rcpf(x)
 #endif
+#ifndef MUGEN_PLAN_SQRT
+#define MUGEN_PLAN_SQRT(x) __builtin_amdgcn_sqrtf(x)
+#endif
 
 namespace mugen_attn {
 
@@ -85,6 +88,17 @@ MUGEN_PLAN_FN int plan_many(int B, int mult, int budget, int c0, int sum, int mx
         if (total(even, plan_rcp(even)) * mult <= budget) return even;
     }
     return plan_grow(c, mx, mult, budget, total);
+}
+
+// MLA decode: the least chunk (units) for `sum` units of R query rows.  A unit is
+// ~0.4 us of a workgroup's time, and a split's partials (R x 512 x 2 bytes there and
+// back) ~0.1 us of the call at 128 rows, so the sum of both is least around
+// sqrt(sum R / 600) (128 heads, caches of 8192, us at 64 / 128 / 192 / 256 tokens: 8
+// sequences of 200..1638 23.3 / 16.9 / 16.4 / 16.9, 4 19.0 / 15.3 / 15.3 / 16.1, 8 of
+// 80..400 13.3 / 13.5 / 14.6 / 15.9).  Less than that: full caches keep their 32 even
+// splits (3 of 8192 tokens 20.3 us at 8 units, 22.4 at 9)
+MUGEN_PLAN_FN int plan_mla_least(int sum, int R) {
+    return plan_max(1, (int)(MUGEN_PLAN_SQRT((float)sum * (float)R * (1.0f / 1400.0f)) + 0.5f));
 }
 
 }  // namespace mugen_attn

@@ -19,6 +19,7 @@ static float host_rcp(float x) {
     return g_ulp == 0 ? r : std::nextafter(r, g_ulp > 0 ? 2.0f * r : 0.0f);
 }
 #define MUGEN_PLAN_RCP(x) host_rcp(x)
+#define MUGEN_PLAN_SQRT(x) std::sqrt(x)
 #include "split_plan.h"
 
 using namespace mugen_attn;
@@ -30,7 +31,7 @@ int exact_ceil(int a, int b) { return (a + b - 1) / b; }
 
 struct Case {
     int kinds, mult, budget, cmin, cap;
-    bool empty_counts;         // an empty sequence still has one split (GQA)
+    bool empty_counts;         // (GQA, where cmin is fixed; else MLA) an empty sequence still has one split
     std::vector<int> T, nq;    // tokens, of which quantised (kinds 2)
     int longest = 1 << 30;     // the longest chunk that is good enough
 };
@@ -58,7 +59,9 @@ void check(const Case& c, const char* what) {
         }
         return n;
     };
-    const int c0 = plan_by_cap(mx, c.cmin, c.cap);
+    // MLA: mult blocks of 64 query rows
+    const int cmin = c.empty_counts ? c.cmin : plan_mla_least(sum, 64 * c.mult);
+    const int c0 = plan_by_cap(mx, cmin, c.cap);
     int chunk;
     if (B <= 8)
         chunk = c.kinds == 1 ? plan_few<1>(B, c.mult, c.budget, c0, c.cap, sum, mx, total)
@@ -77,7 +80,7 @@ void check(const Case& c, const char* what) {
     items *= c.mult;
     // workgroups of the launch: one round, or every slot of every sequence
     const long slots = c.cap + c.kinds - 1, wgs = std::min<long>(c.budget, (long)B * c.mult * slots);
-    if (chunk < c.cmin || items > wgs || most > slots || chunk > c.longest) {
+    if (chunk < cmin || items > wgs || most > slots || chunk > c.longest) {
         violations++;
         if (violations <= 20) {
             std::printf("%s: kinds %d batch %d mult %d budget %d cap %d ulp %d: chunk %d, %ld items for %ld workgroups, "
@@ -97,7 +100,22 @@ void store(std::vector<int> T, int mult, int budget, int cap, int keep, const ch
 
 }  // namespace
 
+// MLA's least chunk: 128 rows, 8 ragged sequences of up to 1638 tokens (64-token
+// chunks there have more partials to merge than tiles to walk), 3 full ones of 8192,
+// whose 32 even splits stay, and a short one
+void least(int sum, int R, int lo, int hi) {
+    const int c = plan_mla_least(sum, R);
+    if (c < lo || c > hi) {
+        violations++;
+        std::printf("least chunk of %d units, %d rows: %d, not %d..%d\n", sum, R, c, lo, hi);
+    }
+}
+
 int main(int argc, char** argv) {
+    least(225, 128, 4, 6);
+    least(768, 128, 1, 8);
+    least(8, 128, 1, 1);
+    least(225, 16, 1, 2);
     std::mt19937 rng(argc > 1 ? (unsigned)std::atoi(argv[1]) : 1u);
     const int draws = argc > 2 ? std::atoi(argv[2]) : 20000;
     auto pick = [&](int lo, int hi) { return (int)(lo + rng() % (unsigned)(hi - lo + 1)); };
